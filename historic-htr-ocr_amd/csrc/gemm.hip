@@ -1,86 +1,14 @@
 // Dense kernels of the prefill for gfx950: Y[M,N] (+)= X[M,K]·Wᵀ with q8_0 weights, RMS norm over rows, SwiGLU.
 //
-// Reference semantics: matmul.wgsl:47-91 (F32 path: W dequantised exactly — q·d is exact in f32 — and f32 fma
-// accumulation; acc = 1 adds onto Y, the residual stream), rms_norm.wgsl:21-41, swiglu.wgsl:18-24 (text.rs:484-518).
-//
-// The GEMM on the matrix cores (k_gemm_q8_0_mfma; N a multiple of 64): v_mfma_f32_32x32x2_f32 keeps the F32 path's
-// f32 products and sums (the order is the matrix unit's). 64×64 output tiles (M is the prompt length, ~1000, so small
-// tiles keep 256+ workgroups busy), 4 waves of one 32×32 MFMA tile each, K in steps of 32 = one q8_0 block: X and the
-// exactly dequantised W tile are staged in LDS as f32 (double-buffered, the next step's global loads in flight),
-// 16-byte chunks placed at chunk ^ (row/2 % 8) so 16 lanes' 16-byte reads fall on 16 bank groups. Lane half h takes
-// the 16 consecutive k of 16h … 16h + 15 over the step's 16 MFMAs (k-slot h of each), so a lane's fragments are 4
-// contiguous 16-byte reads. Measured (1023 rows): see the bench's prefill. Other shapes: k_gemm_q8_0_f32, 64×64
-// tiles, 256 threads with 4×4 outputs each in f32 fma.
-//
-// The f16 compute path (matmul_coop_q8_0 / matmul128h_q8_0, gpu.rs:1976-1995) rounds X and the dequantised W to f16
-// where they enter the tiles and accumulates in f32: k_gemm_q8_0_f32<true> does that for any shape (the MFMA kernels
-// of that path, on f16 planes made by k_q8_to_f16, are in mfma_gemm.hip).
+// Reference semantics: matmul.wgsl:47-91 (F32 path: W dequantised exactly — q·d is exact in f32 — and f32
+// accumulation; acc = 1 adds onto Y, the residual stream), matmul_coop_q8_0 / matmul128h_q8_0 (gpu.rs:1976-1995, the
+// f16 path: X and the dequantised W rounded to f16 where they enter the tiles, f32 accumulation), rms_norm.wgsl:21-41,
+// swiglu.wgsl:18-24 (text.rs:484-518). The prefill's GEMMs on f16 planes made at load are in mfma_gemm.hip.
 #include <algorithm>
 
 #include "htr_internal.h"
 
 namespace {
-
-constexpr int BM = 64, BN = 64, BK = 32;
-
-// R16: X and W values rounded to f16 (round to nearest even) as they enter the tiles
-template <bool R16> __device__ __forceinline__ float tile_val(float v) { return R16 ? (float)(_Float16)v : v; }
-
-template <bool R16>
-__global__ __launch_bounds__(256) void k_gemm_q8_0_f32(const float *x, const int8_t *wq, const _Float16 *wd, float *y,
-                                                       int m, int n, int k, int acc) {
-    __shared__ float s_a[BK][BM + 4];
-    __shared__ float s_b[BK][BN + 4];
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
-    const int nb = k / 32;
-    float c[4][4] = {};
-    for (int k0 = 0; k0 < k; k0 += BK) {
-        // X tile: 64 rows × 32 k (8 per thread, k fastest for coalescing)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int e = tid + 256 * i, r = e / BK, cc = e % BK;
-            const int gr = row0 + r;
-            s_a[cc][r] = gr < m ? tile_val<R16>(x[(size_t)gr * k + k0 + cc]) : 0.0f;
-        }
-        // W tile: 64 columns × 32 quants of one block each, times that block's scale
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int e = tid + 256 * i, r = e / BK, cc = e % BK;
-            const int gc = col0 + r;
-            float v = 0.0f;
-            if (gc < n) v = tile_val<R16>((float)wq[(size_t)gc * k + k0 + cc] * (float)wd[(size_t)gc * nb + k0 / 32]);
-            s_b[cc][r] = v;
-        }
-        __syncthreads();
-#pragma unroll 8
-        for (int kk = 0; kk < BK; kk++) {
-            float a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                a[i] = s_a[kk][ty + 16 * i];
-                b[i] = s_b[kk][tx + 16 * i];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) c[i][j] = fmaf(a[i], b[j], c[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int r = row0 + ty + 16 * i;
-        if (r >= m) continue;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int cc = col0 + tx + 16 * j;
-            if (cc >= n) continue;
-            float *o = y + (size_t)r * n + cc;
-            *o = acc ? *o + c[i][j] : c[i][j];
-        }
-    }
-}
 
 // one workgroup per row: y = x · 1/sqrt(mean(x²) + eps) · w
 __global__ __launch_bounds__(256) void k_rms_norm(const float *x, const float *w, float *y, int dim, float eps) {
@@ -105,71 +33,294 @@ __global__ __launch_bounds__(256) void k_swiglu(float *g, const float *u, size_t
 }
 
 
+// ---- GEMMs on q8_0 weights -------------------------------------------------------------------------------------------
+//
+// One kernel for both compute paths and any shape, on the 16-bit matrix cores:
+//   f16 path  X and f16(q·d) rounded to nearest even as they enter LDS, v_mfma_f32_32x32x16_f16, f32 sums;
+//   F32 path  every product of the exact q8_0 value with the f32 X. A quant is a bf16 value (7 bits) and X is the sum
+//             of three (EX: its top 8 bits, the next 8, the last 8, each truncated, so x = b1 + b2 + b3 exactly), so
+//             three bf16 MFMAs add a block's Σ q·x in f32 with every product exact, and one f32 fma per output and
+//             block adds d·Σ q·x: three 16-bit MFMAs stand for what takes f32 ones sixteen times as long. Exact for
+//             |x| < 2^115 (a block's sum of q·x stays finite where the scaled one does); ±inf and NaN pass as they are.
+// Work: a workgroup owns 64T × 64T outputs; KG groups of 4 waves (2 × 2, 32T × 32T outputs a wave) take the K stages in
+// turn, each through its own pair of LDS buffers, and their sums are added in group order through LDS at the end: a
+// prompt of some hundred rows makes few tiles, and the groups give such a CU four waves a SIMD to hide the loads'
+// latency without a second launch for the sum. A stage is KB blocks of 32 k (f16: 2, EX: 1); its loads go to registers
+// R stages ahead and are converted as they are stored to LDS (16-byte chunks of 8 k, XOR-placed so that the 16 lanes of
+// a fragment read fall on 16 bank groups). K past the last block is zeros, rows past M and columns past N are read clamped and not stored.
+// Bound: the 128 × 128 tile's MFMAs and conversions about even; the 64 × 64 ones by the stages' load latency. Measured
+// against the kernels before it (f32 FMA tiles on the f16 path, v_mfma_f32_32x32x2_f32 on the F32 path), a call: f16
+// 48 × 1024 × 2048 231 → 13.4 µs, 1925 × 3072 × 1024 422 → 30.4 µs (399 TFLOP/s); F32 1023 × 1024 × 3072 onto the
+// residual 111 → 36 µs (179 TFLOP/s, past the f32 MFMA's 157 peak). Error against 64 bits 5.6e-7 … 9.8e-7 → 1.2e-7 …
+// 2.0e-7: a block's 96 products are summed inside the matrix unit before the one f32 fma that scales them.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ int mf_slot(int r, int q) { return 8 * r + (q ^ ((r >> 1) & 7)); }
+// the slot of chunk c of row r in rows of CPR chunks; the XOR is its own inverse
+template <int CPR> __device__ __forceinline__ int q8_slot(int r, int c) {
+    return CPR * r + (c ^ (CPR == 4 ? (r >> 2) & 3 : (r >> 1) & 7));
+}
 
-__global__ __launch_bounds__(256) void k_gemm_q8_0_mfma(const float *x, const int8_t *wq, const _Float16 *wd, float *y,
-                                                        int m, int n, int k, int acc) {
-    __shared__ __attribute__((aligned(16))) float4 s_a[2][64 * 8];  // [row][chunk] f32, 8 KB a buffer
-    __shared__ __attribute__((aligned(16))) float4 s_b[2][64 * 8];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-    const int row0 = blockIdx.y * 64, col0 = blockIdx.x * 64;
-    const int nb = k / 32;
-    // staging: thread t moves row t/4, k 8·(t%4) … + 7 of the X tile and of the W tile
-    const int lr = tid >> 2, lq = tid & 3;
-    const float *xr = x + (size_t)min(row0 + lr, m - 1) * k + 8 * lq;
-    const int8_t *wr = wq + (size_t)(col0 + lr) * k + 8 * lq;
-    const _Float16 *dr = wd + (size_t)(col0 + lr) * nb;
-    float4 ra0, ra1;
-    int2 rq;
-    float rd;
-    auto gload = [&](int kb) {
-        const float4 *xs = reinterpret_cast<const float4 *>(xr + 32 * kb);
-        ra0 = xs[0];
-        ra1 = xs[1];
-        rq = *reinterpret_cast<const int2 *>(wr + 32 * kb);
-        rd = (float)dr[kb];
-    };
-    auto lstore = [&](int buf) {
-        s_a[buf][mf_slot(lr, 2 * lq)] = ra0;
-        s_a[buf][mf_slot(lr, 2 * lq + 1)] = ra1;
-        const uint32_t u0 = (uint32_t)rq.x, u1 = (uint32_t)rq.y;
-        s_b[buf][mf_slot(lr, 2 * lq)] = make_float4((float)(int8_t)u0 * rd, (float)(int8_t)(u0 >> 8) * rd,
-                                                    (float)(int8_t)(u0 >> 16) * rd, (float)(int8_t)(u0 >> 24) * rd);
-        s_b[buf][mf_slot(lr, 2 * lq + 1)] = make_float4((float)(int8_t)u1 * rd, (float)(int8_t)(u1 >> 8) * rd,
-                                                        (float)(int8_t)(u1 >> 16) * rd, (float)(int8_t)(u1 >> 24) * rd);
-    };
-    f32x16 c;
+// the high halves of two words as one: (hi16(a), hi16(b)), a in the low half
+__device__ __forceinline__ uint32_t hi_pair(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+
+__device__ __forceinline__ int8_t q_byte(int2 v, int e) { return (int8_t)((uint32_t)(e < 4 ? v.x : v.y) >> (8 * (e & 3))); }
+
+// 8 values as three bf16 pieces, x = b1 + b2 + b3: each piece the top 16 bits of what is left (no rounding: 24 = 3 · 8
+// bits). ±inf and NaN: the value itself and two zeros (inf − inf would make NaN of an infinity)
+__device__ __forceinline__ void split3(const float (&x)[8], int4 (&out)[3]) {
+    uint32_t b[3][8];
+    bool odd = false;
 #pragma unroll
-    for (int r = 0; r < 16; r++) c[r] = 0.0f;
-    const int fr_a = wm * 32 + (lane & 31), fr_b = wn * 32 + (lane & 31), h = lane >> 5;
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    for (int kb = 0; kb < nb; kb++) {
-        const int cur = kb & 1;
-        if (kb + 1 < nb) gload(kb + 1);
-        float a[16], b[16];
+    for (int e = 0; e < 8; e++) {
+        b[0][e] = __float_as_uint(x[e]);
+        const float r1 = x[e] - __uint_as_float(b[0][e] & 0xffff0000u);
+        b[1][e] = __float_as_uint(r1);
+        b[2][e] = __float_as_uint(r1 - __uint_as_float(b[1][e] & 0xffff0000u));
+        odd |= !(fabsf(x[e]) <= 3.4028235e38f);
+    }
+    if (__builtin_expect(odd, 0)) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const float4 va = s_a[cur][mf_slot(fr_a, 4 * h + q)], vb = s_b[cur][mf_slot(fr_b, 4 * h + q)];
-            a[4 * q] = va.x, a[4 * q + 1] = va.y, a[4 * q + 2] = va.z, a[4 * q + 3] = va.w;
-            b[4 * q] = vb.x, b[4 * q + 1] = vb.y, b[4 * q + 2] = vb.z, b[4 * q + 3] = vb.w;
+        for (int e = 0; e < 8; e++)
+            if (!(fabsf(x[e]) <= 3.4028235e38f)) {
+                if (x[e] != x[e]) b[0][e] |= 0x00400000u;  // a NaN whose payload sits in the low half stays one
+                b[1][e] = b[2][e] = 0u;
+            }
+    }
+#pragma unroll
+    for (int s = 0; s < 3; s++)
+        out[s] = make_int4((int)hi_pair(b[s][0], b[s][1]), (int)hi_pair(b[s][2], b[s][3]),
+                           (int)hi_pair(b[s][4], b[s][5]), (int)hi_pair(b[s][6], b[s][7]));
+}
+
+template <bool EX, int T, int KG> struct Q8Tile {
+    static constexpr int BT = 64 * T, KB = EX ? 1 : 2, CPR = 4 * KB, PL = EX ? 3 : 1, R = 2;
+    static constexpr int UN = T * KB;                                  // chunks a thread stages of X, and of W
+    static constexpr int ACH = PL * BT * CPR, BUF = ACH + BT * CPR;    // 16-byte chunks: X's planes, a buffer
+    static constexpr int LDS = 2 * KG * BUF;
+    static_assert(KG == 1 || 2 * BUF * 16 >= BT * BT * 4, "a group's sums fit its buffers");
+};
+
+// al: X may be read in 16-byte units
+template <bool EX, int T, int KG>
+__global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const int8_t *wq, const _Float16 *wd, float *y,
+                                                        int m, int n, int k, int acc, int al, int tiles_m, int tiles_n) {
+    using C = Q8Tile<EX, T, KG>;
+    constexpr int KB = C::KB, CPR = C::CPR, R = C::R, UN = C::UN;
+    __shared__ __attribute__((aligned(16))) int4 s_t[C::LDS];
+    __shared__ float s_d[EX ? KG : 1][2][EX ? C::BT : 1];
+    const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8), tid = threadIdx.x & 255, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+    // workgroup b runs on XCD b mod 8: each XCD takes a contiguous band of tiles, walked 4 tile rows at a time, so the
+    // workgroups of an XCD share X and W rows in its L2
+    int tm, tn;
+    {
+        const int total = tiles_m * tiles_n, xcd = (int)blockIdx.x % 8, i = (int)blockIdx.x / 8;
+        const int t = xcd * (total / 8) + min(xcd, total % 8) + i, gsz = 4 * tiles_n, g = t / gsz, gr = t % gsz;
+        const int gm = min(4, tiles_m - 4 * g);
+        tm = 4 * g + gr % gm;
+        tn = gr / gm;
+    }
+    const int row0 = tm * C::BT, col0 = tn * C::BT, nb = k / 32, nst = (nb + KB - 1) / KB;
+    int4 *buf0 = s_t + grp * 2 * C::BUF;
+
+    // staging: chunk u = tid + 256·i of the stage is row u / CPR, k 8·(u % CPR) … + 7, of the X tile and of the W tile
+    struct Regs {
+        float4 a[UN][2];
+        int2 q[UN];
+        _Float16 d[UN];
+    } ring[R];
+    auto gload = [&](Regs &r, int st) {
+#pragma unroll
+        for (int i = 0; i < UN; i++) {
+            const int u = tid + 256 * i, rr = u / CPR, c = u % CPR, b = min(st * KB + c / 4, nb - 1);
+            const float *xs = x + (size_t)min(row0 + rr, m - 1) * k + 32 * b + 8 * (c & 3);
+            if (al) {
+                r.a[i][0] = reinterpret_cast<const float4 *>(xs)[0];
+                r.a[i][1] = reinterpret_cast<const float4 *>(xs)[1];
+            } else {
+                r.a[i][0] = make_float4(xs[0], xs[1], xs[2], xs[3]);
+                r.a[i][1] = make_float4(xs[4], xs[5], xs[6], xs[7]);
+            }
+            const size_t wr = min(col0 + rr, n - 1);
+            r.q[i] = *reinterpret_cast<const int2 *>(wq + wr * k + 32 * b + 8 * (c & 3));
+            r.d[i] = wd[wr * nb + b];
+        }
+    };
+    auto lstore = [&](const Regs &r, int st, int buf) {
+        int4 *s = buf0 + buf * C::BUF;
+#pragma unroll
+        for (int i = 0; i < UN; i++) {
+            const int u = tid + 256 * i, rr = u / CPR, c = u % CPR, at = q8_slot<CPR>(rr, c);
+            const bool in = st * KB + c / 4 < nb;
+            const float4 a0 = r.a[i][0], a1 = r.a[i][1];
+            float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+            if (!in) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = 0.0f;
+            }
+            const float d = in ? (float)r.d[i] : 0.0f;
+            if constexpr (EX) {
+                int4 p[3];
+                split3(v, p);
+#pragma unroll
+                for (int t = 0; t < 3; t++) s[t * C::BT * CPR + at] = p[t];
+                uint32_t f[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) f[e] = __float_as_uint((float)q_byte(r.q[i], e));
+                s[C::ACH + at] = make_int4((int)hi_pair(f[0], f[1]), (int)hi_pair(f[2], f[3]),
+                                           (int)hi_pair(f[4], f[5]), (int)hi_pair(f[6], f[7]));
+                if (c == 0) s_d[grp][buf][rr] = d;
+            } else {
+                half2_t hx[4], hw[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    hx[e] = __builtin_convertvector((float2_t{v[2 * e], v[2 * e + 1]}), half2_t);
+                    hw[e] = __builtin_convertvector(
+                        (float2_t{(float)q_byte(r.q[i], 2 * e) * d, (float)q_byte(r.q[i], 2 * e + 1) * d}), half2_t);
+                }
+                int4 px, pw;
+                __builtin_memcpy(&px, hx, 16);
+                __builtin_memcpy(&pw, hw, 16);
+                s[at] = px;
+                s[C::ACH + at] = pw;
+            }
+        }
+    };
+    f32x16 c[T][T];
+#pragma unroll
+    for (int i = 0; i < T; i++)
+#pragma unroll
+        for (int j = 0; j < T; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) c[i][j][r] = 0.0f;
+    const int fa = 32 * T * wm + (lane & 31), fb = 32 * T * wn + (lane & 31), hk = lane >> 5;
+    auto compute = [&](int buf) {
+        const int4 *s = buf0 + buf * C::BUF;
+        if constexpr (EX) {
+            f32x16 p[T][T];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                bf16x8 b[T];
+#pragma unroll
+                for (int j = 0; j < T; j++)
+                    b[j] = *reinterpret_cast<const bf16x8 *>(s + C::ACH + q8_slot<CPR>(fb + 32 * j, 2 * h + hk));
+#pragma unroll
+                for (int pl = 0; pl < 3; pl++) {
+                    bf16x8 a[T];
+#pragma unroll
+                    for (int i = 0; i < T; i++)
+                        a[i] = *reinterpret_cast<const bf16x8 *>(s + pl * C::BT * CPR + q8_slot<CPR>(fa + 32 * i, 2 * h + hk));
+#pragma unroll
+                    for (int i = 0; i < T; i++)
+#pragma unroll
+                        for (int j = 0; j < T; j++)
+                            p[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], h + pl ? p[i][j] : f32x16{}, 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < T; j++) {
+                const float d = s_d[grp][buf][fb + 32 * j];
+#pragma unroll
+                for (int i = 0; i < T; i++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) c[i][j][r] = fmaf(p[i][j][r], d, c[i][j][r]);
+            }
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2 * KB; h++) {
+                half8 a[T], b[T];
+#pragma unroll
+                for (int i = 0; i < T; i++) a[i] = *reinterpret_cast<const half8 *>(s + q8_slot<CPR>(fa + 32 * i, 2 * h + hk));
+#pragma unroll
+                for (int j = 0; j < T; j++)
+                    b[j] = *reinterpret_cast<const half8 *>(s + C::ACH + q8_slot<CPR>(fb + 32 * j, 2 * h + hk));
+#pragma unroll
+                for (int i = 0; i < T; i++)
+#pragma unroll
+                    for (int j = 0; j < T; j++) c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[j], c[i][j], 0, 0, 0);
+            }
+        }
+    };
+    // the barrier between a buffer's stores and its reads: LDS accesses done, the register loads left in flight
+    auto lds_barrier = [&] {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // group grp's stage i is grp + KG·i; every group runs the same count (a stage past the last is zeros). Step i reads
+    // buffer i % 2 while stage i + 1 is stored to the other, which step i − 1 read before the barrier that ended it
+    const int steps = (nst + KG - 1) / KG;
+#pragma unroll
+    for (int r = 0; r < R; r++) gload(ring[r], grp + KG * r);
+    lstore(ring[0], grp, 0);
+    gload(ring[0], grp + KG * R);
+    lds_barrier();
+    for (int i0 = 0; i0 < steps; i0 += R) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int i = i0 + r;
+            if (i < steps) {
+                compute(i & 1);
+                if (i + 1 < steps) lstore(ring[(r + 1) % R], grp + KG * (i + 1), (i + 1) & 1);
+                gload(ring[(r + 1) % R], grp + KG * (i + 1 + R));
+                lds_barrier();
+            }
+        }
+    }
+    // lane ℓ, register r: row 8(r/4) + 4(ℓ/32) + r%4, column ℓ%32 of each 32 × 32 tile
+    if constexpr (KG == 1) {
+#pragma unroll
+        for (int j = 0; j < T; j++) {
+            const int col = col0 + fb + 32 * j;
+#pragma unroll
+            for (int i = 0; i < T; i++) {
+                const int rbase = row0 + 32 * T * wm + 32 * i + 4 * hk;
+                float old[16];
+                if (acc) {  // every load before the first store, which may alias them
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        old[r] = y[(size_t)min(rbase + 8 * (r >> 2) + (r & 3), m - 1) * n + min(col, n - 1)];
+                }
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int row = rbase + 8 * (r >> 2) + (r & 3);
+                    if (row < m && col < n) y[(size_t)row * n + col] = acc ? old[r] + c[i][j][r] : c[i][j][r];
+                }
+            }
+        }
+    } else {
+        // the groups' sums through their own (idle) buffers, added in group order
+        constexpr int BT = C::BT, GS = 2 * C::BUF * 4;  // floats from a group's buffers to the next's
+        float *s_o = reinterpret_cast<float *>(s_t);
+#pragma unroll
+        for (int i = 0; i < T; i++)
+#pragma unroll
+            for (int j = 0; j < T; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    s_o[grp * GS + (32 * T * wm + 32 * i + 8 * (r >> 2) + 4 * hk + (r & 3)) * BT + fb + 32 * j] = c[i][j][r];
+        __syncthreads();
+        constexpr int NE = BT * BT / (256 * KG);
+        float old[NE];
+        if (acc) {  // every load before the first store, which may alias them
+#pragma unroll
+            for (int e = 0; e < NE; e++) {
+                const int o = threadIdx.x + 256 * KG * e;
+                old[e] = y[(size_t)min(row0 + o / BT, m - 1) * n + min(col0 + o % BT, n - 1)];
+            }
         }
 #pragma unroll
-        for (int s2 = 0; s2 < 16; s2++) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s2], b[s2], c, 0, 0, 0);
-        if (kb + 1 < nb) lstore(cur ^ 1);
-        __syncthreads();
-    }
-    const int col = col0 + wn * 32 + (lane & 31);
+        for (int e = 0; e < NE; e++) {
+            const int o = threadIdx.x + 256 * KG * e, row = row0 + o / BT, col = col0 + o % BT;
+            float v = s_o[o];
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int row = row0 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row >= m) continue;
-        float *o = y + (size_t)row * n + col;
-        *o = acc ? *o + c[r] : c[r];
+            for (int g = 1; g < KG; g++) v += s_o[g * GS + o];
+            if (row < m && col < n) y[(size_t)row * n + col] = acc ? old[e] + v : v;
+        }
     }
 }
 
@@ -202,27 +353,36 @@ int weight_attach_f16(htr_device *dev, hipStream_t st, htr_weight *w) {
     return htr_launched(dev, "k_q8_to_f16");
 }
 
+namespace {
+
+template <bool EX, int T, int KG>
+int launch_q8(htr_device *dev, hipStream_t st, const float *x, const htr_weight *w, float *y, int m, int acc) {
+    const int n = (int)w->rows, bt = 64 * T, tm = (m + bt - 1) / bt, tn = (n + bt - 1) / bt;
+    hipLaunchKernelGGL((k_gemm_q8_0<EX, T, KG>), dim3(tm * tn), dim3(256 * KG), 0, st, x, w->q, w->d, y, m, n,
+                       (int)w->cols, acc, (int)((uintptr_t)x % 16 == 0), tm, tn);
+    return 0;
+}
+
+template <bool EX> int gemm_q8(htr_device *dev, hipStream_t st, const float *x, const htr_weight *w, float *y, int m, int acc) {
+    if (!w->q) return htr_fail("gemm: weight has no q8_0 planes");
+    const int n = (int)w->rows;
+    const long t128 = (long)((m + 127) / 128) * ((n + 127) / 128), t64 = (long)((m + 63) / 64) * ((n + 63) / 64);
+    if (t128 >= dev->n_cu) launch_q8<EX, 2, 1>(dev, st, x, w, y, m, acc);
+    else if (t64 >= 2 * dev->n_cu) launch_q8<EX, 1, 2>(dev, st, x, w, y, m, acc);
+    else launch_q8<EX, 1, 4>(dev, st, x, w, y, m, acc);
+    return htr_launched(dev, EX ? "k_gemm_q8_0<f32>" : "k_gemm_q8_0<f16>");
+}
+
+}  // namespace
+
 int launch_gemm_q8_0_f32(htr_device *dev, hipStream_t st, const float *x, const htr_weight *w, float *y, int m,
                          int acc) {
-    if (!w->q) return htr_fail("gemm: weight has no q8_0 planes");
-    dim3 grid(((int)w->rows + BN - 1) / BN, (m + BM - 1) / BM);
-    if (w->rows % 64 == 0 && w->cols % 32 == 0) {
-        hipLaunchKernelGGL(k_gemm_q8_0_mfma, grid, dim3(256), 0, st, x, w->q, w->d, y, m, (int)w->rows, (int)w->cols,
-                           acc);
-        return htr_launched(dev, "k_gemm_q8_0_mfma");
-    }
-    hipLaunchKernelGGL(k_gemm_q8_0_f32<false>, grid, dim3(256), 0, st, x, w->q, w->d, y, m, (int)w->rows,
-                       (int)w->cols, acc);
-    return htr_launched(dev, "k_gemm_q8_0_f32");
+    return gemm_q8<true>(dev, st, x, w, y, m, acc);
 }
 
 int launch_gemm_q8_0_r16(htr_device *dev, hipStream_t st, const float *x, const htr_weight *w, float *y, int m,
                          int acc) {
-    if (!w->q) return htr_fail("gemm: weight has no q8_0 planes");
-    dim3 grid(((int)w->rows + BN - 1) / BN, (m + BM - 1) / BM);
-    hipLaunchKernelGGL(k_gemm_q8_0_f32<true>, grid, dim3(256), 0, st, x, w->q, w->d, y, m, (int)w->rows,
-                       (int)w->cols, acc);
-    return htr_launched(dev, "k_gemm_q8_0_f32<r16>");
+    return gemm_q8<false>(dev, st, x, w, y, m, acc);
 }
 
 int launch_rms_norm(htr_device *dev, hipStream_t st, const float *x, const float *w, float *y, int rows, int dim,

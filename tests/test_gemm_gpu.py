@@ -223,6 +223,80 @@ def test_matmul_q8_0_on_both_compute_paths(dev, m, n, k):
     w.free()
 
 
+class _At:
+    """a buffer's memory from a byte offset on, as the entry points take it"""
+
+    def __init__(self, buf, off):
+        self.ptr = buf.ptr + off
+
+
+def _deq64(blocks, n, k):
+    b = blocks.reshape(n, k // 32, 34)
+    return (b[:, :, 2:].view(np.int8).astype(np.float64) * b[:, :, :2].copy().view(np.float16).astype(np.float64)).reshape(n, k)
+
+
+# one block, odd block counts, tiles of 64 and 128 cut on both sides; the tile counts on either side of the launch's
+# rules (4 K groups, 2 K groups, 128 × 128 tiles); X off the 16-byte grid
+@pytest.mark.parametrize("m,n,k,off", [(1, 1, 32, 0), (1, 65, 96, 4), (63, 129, 160, 0), (64, 64, 64, 8), (65, 63, 1024, 0),
+                                       (333, 1000, 3072, 0), (1025, 2000, 224, 0), (2050, 2049, 96, 0), (2050, 2049, 64, 4)])
+def test_matmul_q8_0_tiles_against_fp64(dev, m, n, k, off):
+    """every output within the f32 rounding of its own sum: K/32 block sums added one by one (and, on the F32 path, a
+    block's 3 · 32 exact products before them; on the f16 path the K products)"""
+    blocks = htr.synth_q8_0(5 * m + n + k, n, k)
+    x = (htr.synth_normal(m + 7 * k, m * k) * np.exp(htr.synth_normal(m + 9 * k, m * k))).astype(np.float32).reshape(m, k)
+    base = htr.synth_normal(12, m * n).reshape(m, n)
+    w, w64 = htr.Weight(dev, blocks, n, k), _deq64(blocks, n, k)
+    xb = dev.alloc(m * k * 4 + 16)
+    htr._check(htr.lib().htr_upload(dev.h, xb.ptr + off, htr._ptr(x), x.nbytes))
+    keep = dev.compute
+    try:
+        for path in (htr.COMPUTE_F32, htr.COMPUTE_F16):
+            dev.compute = path
+            half = path == htr.COMPUTE_F16
+            xx = (x.astype(np.float16) if half else x).astype(np.float64)
+            ww = w64.astype(np.float16).astype(np.float64) if half else w64
+            want, terms = xx @ ww.T, (k if half else k // 32 + 96) + 2
+            bound = terms * 2.0 ** -24 * (np.abs(xx) @ np.abs(ww).T) + 2.0 ** -23 * np.abs(base)
+            for acc in (False, True):
+                y = dev.upload(base)
+                htr.matmul_q8_0(dev, _At(xb, off), m, w, y, acc=acc)
+                err = np.abs(y.download(np.float32).reshape(m, n) - (want + base if acc else want))
+                assert np.all(err <= bound), (path, acc, float(np.max(err / bound)))
+                y.free()
+    finally:
+        dev.compute = keep
+    xb.free()
+    w.free()
+
+
+def test_matmul_q8_0_f32_path_keeps_infinities_and_nans(dev):
+    """one infinity a row gives ±inf (NaN where its quant is 0), a NaN a NaN — also one whose payload is in its low
+    half — and the largest finite values stay exact; the other rows are untouched"""
+    m, n, k = 6, 70, 128
+    blocks = htr.synth_q8_0(77, n, k).reshape(n, k // 32, 34).copy()
+    blocks[5, 1, 2 + 3] = 0  # the quant of k = 35 in row 5
+    x = htr.synth_normal(78, m * k).reshape(m, k)
+    x[0, 35], x[1, 35], x[2, 64] = np.inf, -np.inf, np.nan
+    x[3, 7] = np.array([0x7F800001], np.uint32).view(np.float32)[0]
+    x[4, 100] = np.float32(2.0 ** 100)
+    w, xb = htr.Weight(dev, blocks.reshape(-1), n, k), dev.upload(x)
+    y, keep = dev.alloc(m * n * 4), dev.compute
+    try:
+        dev.compute = htr.COMPUTE_F32
+        htr.matmul_q8_0(dev, xb, m, w, y)
+        got = y.download(np.float32).reshape(m, n)
+    finally:
+        dev.compute = keep
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ _deq64(blocks.reshape(-1), n, k).T
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    assert np.isnan(got[2:4]).all() and np.isnan(got[0, 5]) and np.isinf(got[0, 6])
+    assert np.array_equal(np.sign(got[np.isinf(got)]), np.sign(want[np.isinf(want)]))
+    np.testing.assert_allclose(got[ok], want[ok], rtol=1e-4, atol=1e-4)
+    w.free()
+
+
 def test_compute_path_setting(dev):
     keep = dev.compute
     assert keep in (htr.COMPUTE_F32, htr.COMPUTE_F16)
