@@ -6,6 +6,8 @@
 //
 // KV cache layout (this library's): f16, head-major per layer, [n_kv][n_ctx][128] — one KV head's keys are
 // contiguous, so a workgroup working on (kv head, key chunk) reads one contiguous range (256 bytes per key).
+#include <type_traits>
+
 #include "htr_internal.h"
 #include "wave.h"
 
@@ -48,35 +50,6 @@ __global__ __launch_bounds__(64) void k_qkv_post(float *qkv, const float *qn, co
         _Float16 *o = kc + ((size_t)(h - n_head) * n_ctx + pos) * D;
         o[lane] = (_Float16)x0;
         o[lane + 64] = (_Float16)x1;
-    }
-}
-
-// prefill rows: block (t, h): q heads, k heads (→ f16 cache rows pos0 + t), v heads (→ f16 cache)
-__global__ __launch_bounds__(64) void k_qk_rows(float *q, float *k, const float *v, const float *qn, const float *kn,
-                                                const float *rope, int n_head, int n_kv, int pos0, int n_ctx,
-                                                float eps, _Float16 *kc, _Float16 *vc) {
-    const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-    const int pos = pos0 + t;
-    if (h < n_head) {
-        float *x = q + ((size_t)t * n_head + h) * D;
-        float x0 = x[lane], x1 = x[lane + 64];
-        norm_rope(x0, x1, qn, rope + (size_t)pos * D, lane, eps);
-        x[lane] = x0;
-        x[lane + 64] = x1;
-    } else if (h < n_head + n_kv) {
-        const int j = h - n_head;
-        float *x = k + ((size_t)t * n_kv + j) * D;
-        float x0 = x[lane], x1 = x[lane + 64];
-        norm_rope(x0, x1, kn, rope + (size_t)pos * D, lane, eps);
-        _Float16 *o = kc + ((size_t)j * n_ctx + pos) * D;
-        o[lane] = (_Float16)x0;
-        o[lane + 64] = (_Float16)x1;
-    } else {
-        const int j = h - n_head - n_kv;
-        const float *x = v + ((size_t)t * n_kv + j) * D;
-        _Float16 *o = vc + ((size_t)j * n_ctx + pos) * D;
-        o[lane] = (_Float16)x[lane];
-        o[lane + 64] = (_Float16)x[lane + 64];
     }
 }
 
@@ -191,6 +164,31 @@ __device__ __forceinline__ void post_apply(const PostIn &p, const float (&cs)[16
         const float c = cs[2 * e], s = cs[2 * e + 1];
         out[e] = j < 8 ? ya * c - yb * s : yb * s + ya * c;
     }
+}
+
+// prefill rows: k heads (norm, RoPE → f16 cache rows pos0 + t) and v heads (→ f16 cache), 16 lanes × 8 dims a head row
+// (the q heads are normed and turned where the causal attention reads them)
+__global__ __launch_bounds__(256) void k_kv_rows(const float *k, const float *v, const float *kn, const float *rope,
+                                                 int n_rows, int n_kv, int pos0, int n_ctx, float eps, _Float16 *kc,
+                                                 _Float16 *vc) {
+    const int lane = threadIdx.x & 63, j = lane & 15, id = blockIdx.x * 16 + (threadIdx.x >> 4);
+    const int row = min(id, n_rows - 1), t = row / (2 * n_kv), h = row % (2 * n_kv), pos = pos0 + t;
+    const bool isv = h >= n_kv;
+    const int kvh = isv ? h - n_kv : h;
+    PostIn in;
+    post_load(in, (isv ? v : k) + ((size_t)t * n_kv + kvh) * D, kn, j);
+    float cs[16], y[8], raw[8];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float4 r = *reinterpret_cast<const float4 *>(rope + (size_t)pos * D + 16 * (j & 7) + 4 * i);
+        cs[4 * i] = r.x, cs[4 * i + 1] = r.y, cs[4 * i + 2] = r.z, cs[4 * i + 3] = r.w;
+    }
+    post_apply(in, cs, j, lane, eps, y);
+    unpack4x2(in.a, raw);
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = isv ? raw[e] : y[e];
+    if (id < n_rows)
+        *reinterpret_cast<int4 *>((isv ? vc : kc) + ((size_t)kvh * n_ctx + pos) * D + 8 * j) = pack8(y);
 }
 
 // FUSED: q is the raw [q | k | v] row of the qkv matvec and the kernel does qkv_post's work itself: each workgroup
@@ -458,213 +456,318 @@ __global__ __launch_bounds__(AW) void k_attn_decode(const float *q, const _Float
 // ---- prefill causal attention ----------------------------------------------------------------------------------------
 //
 // attention_causal.wgsl's arithmetic (text.rs:484-499; the same on every compute path): q·scale in f32, scores as
-// f32 dot products with the f16 keys, an online softmax in f32 from a running max of −3e38 over the keys each query
-// sees (0 … its position), out = acc · (1 / l). Here on the f16 matrix cores (v_mfma_f32_16x16x32_f16) with f32-grade
-// operands: q·scale = qh + ql and p·2^14 = ph + pl, each half rounded to f16 (the pair holds 22 bits; K and V are f16
-// already), so every product is exact and every sum f32; the 2^14 (exact) keeps small p out of f16's subnormals and
-// comes off with 1/l at the end.
+// f32 dot products with the f16 keys, an online softmax in f32 over the keys each query sees (0 … its position),
+// out = acc · (1 / l). Here on the f16 matrix cores (v_mfma_f32_32x32x16_f16) with f32-grade operands: q·scale =
+// qh + ql and p·2^10 = ph + pl, each half rounded to f16 (the pair holds 22 bits; K and V are f16 already), so every
+// product is exact and every sum f32; the 2^10 (exact) keeps small p out of f16's subnormals and drops out with l,
+// which carries it too.
 //
-//   blocks   a pre-pass (k_kv_blocks) copies the keys 0 … n_keys − 1 of each KV head into blocks of 32 keys, 16 KB each,
-//            laid out as LDS holds them: K [32 keys][128 dims] with row r's 16-byte chunk c at 16r + (c ^ r%16), then
-//            Vᵀ [128 dims][32 keys] with row d's chunk g at 512 + 4d + (g ^ (d/4)%4), the keys of chunk g in the order
-//            the P·V MFMA consumes them: 4g … 4g+3, 16 + 4g … 16 + 4g + 3 (the keys lane group g holds in its two
-//            score tiles) — so 16 lanes' fragment reads fall on 16 bank groups and a stage is a plain copy;
-//   work     a workgroup takes 16 queries (one query block) of both q heads of a KV head: 4 waves = 2 heads × 2 halves
-//            of the key blocks (even / odd), the two halves merged through LDS at the end. Stages of 2 blocks go
-//            global → LDS by direct loads, the next stage in flight while one is used. Workgroup j takes query block
-//            n_qb − 1 − j/n_kv for the first half of the grid and j/n_kv − half for the second, so the two workgroups
-//            a CU holds have complementary lengths;
-//   scores   Sᵀ (16 keys × 16 queries) = K·(qh + ql)ᵀ: lane ℓ = 16g + c holds query c's scores of keys 4g … 4g + 3 of
-//            each 16-key tile; the max and the sum over a query's keys are one swap across lane bits 4 and 5 each;
-//   values   Oᵀ (128 dims × 16 queries) += Vᵀ·(ph + pl)ᵀ, the P operand straight from the lane's score registers,
-//            lane ℓ accumulating dims 16t + 4g … of query c, so the rescale by the query's correction stays in the lane.
-constexpr int CQ = 16, CK = 32, CB_CHUNKS = 1024;  // queries a block, keys a block, 16-byte chunks a key block
-constexpr float P_SCALE = 16384.0f, P_UNSCALE = 1.0f / 16384.0f;
+//   work     a workgroup takes 32 queries of both q heads of a KV head: 4 waves = 2 heads × the even / odd key blocks,
+//            the two parts merged through LDS at the end. A stage is 2 blocks of 32 keys (32 KB), K and V each
+//            double-buffered, K a stage ahead of V: the score MFMAs of the next stage run under the softmax of this one.
+//            Two workgroups a CU; the first half of the grid takes the query blocks longest first, the second half
+//            shortest first, so the two that a CU holds have complementary lengths;
+//   blocks   K [32 keys][128 dims] with row r's 16-byte chunk c at 16r + (c ^ r%16), then V [32 keys][128 dims] with
+//            chunk c at 16r + (c ^ 2(r%8)), straight from the cache rows by direct-to-LDS loads (a wave's instruction
+//            is 4 whole rows): 16 lanes' fragment reads of K (16 rows, one chunk) and of V (4 rows, two chunks) fall
+//            on different bank groups. Keys past the last read the last key and are masked;
+//   scores   Sᵀ (32 keys × 32 queries) = K·(qh + ql)ᵀ: lane ℓ = 32h + c holds query c's scores of keys
+//            8(i / 4) + 4h + i % 4 (i < 16); the max over a query's keys is one swap across lane bit 5;
+//   softmax  p = 2^(s·log2 e + nm), nm = 10 − log2 e · (the max when it was last moved): one fma and one v_exp_f32 a
+//            score, and nm is the only state, so its rounding cancels between p, l and O. nm moves (and O and l are
+//            rescaled) only when some p would pass 2^15, so most blocks skip the 64-register rescale;
+//   values   Oᵀ (128 dims × 32 queries) += Vᵀ·(ph + pl)ᵀ: the Vᵀ operand by ds_read_b64_tr_b16 (16 lanes read 4 key
+//            rows × 16 dims and each gets one dim's 4 keys), the P operand straight from the lane's score registers.
+//
+// Bound: the score MFMAs with the softmax between them (a 32x32x16 MFMA takes 17 ns a SIMD here; with its 5 VALU
+// instructions and exponential about 23), then the stage's loads (20 %: a timing copy without them ran 34 µs for 40) and
+// a stage's barrier. Measured against 16 queries a workgroup on 16x16x32 MFMAs, O rescaled at every block and the keys
+// copied into blocks by a launch before it (n_q from position 0, 16 / 8 heads, µs a kernel): 333 queries 11.5 + 4.9 →
+// 10.5, 1023 26.0 + 5.5 → 21.9, 1925 75.6 + 8.1 → 40.5 (375 TFLOP/s of q·k and p·v). Eight waves and four key parts, one
+// workgroup a CU: 13.7, 23.4, 48.6 (its merge is twice the LDS traffic and its waves run in step); only 32 queries on
+// 2000 earlier keys gained, 31.4 → 29.7.
+constexpr int CQ = 32, CK = 32, CB_CHUNKS = 1024;  // queries a workgroup, keys a block, 16-byte chunks a key block
+constexpr int CKS = 2, CW = 64 * 2 * CKS;          // key parts; threads
+constexpr float P_SHIFT = 10.0f, P_TOP = 15.0f;    // log2 of the largest p when nm moves, and before it must
+constexpr float LOG2E = 1.4426950408889634f;
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef __fp16 fp16x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ int kb_kslot(int r, int c) { return 16 * r + (c ^ (r & 15)); }
-__device__ __forceinline__ int kb_vslot(int d, int g) { return 512 + 4 * d + (g ^ ((d >> 2) & 3)); }
-// the key of chunk slot j (0 … 7) of Vᵀ chunk g
-__device__ __forceinline__ int kb_vkey(int g, int j) { return j < 4 ? 4 * g + j : 16 + 4 * g + (j - 4); }
-
-// grid (n_blk, n_kv), 256 threads, 4 chunks a thread; keys ≥ n_keys are zeros (masked wherever they are read)
-__global__ __launch_bounds__(256) void k_kv_blocks(const _Float16 *kc, const _Float16 *vc, int n_ctx, int n_keys,
-                                                   int4 *out) {
-    const int kb = blockIdx.x, kvh = blockIdx.y, n_blk = gridDim.x;
-    const _Float16 *kh = kc + (size_t)kvh * n_ctx * D, *vh = vc + (size_t)kvh * n_ctx * D;
-    int4 *ob = out + ((size_t)kvh * n_blk + kb) * CB_CHUNKS;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int u = threadIdx.x + 256 * i;
-        int4 v = make_int4(0, 0, 0, 0);
-        if (u < 512) {
-            const int r = u >> 4, c = (u & 15) ^ (r & 15), key = CK * kb + r;
-            if (key < n_keys) v = *reinterpret_cast<const int4 *>(kh + (size_t)key * D + 8 * c);
-        } else {
-            const int w = u - 512, d = w >> 2, g = (w & 3) ^ ((d >> 2) & 3);
-            _Float16 e[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int key = CK * kb + kb_vkey(g, j);
-                e[j] = key < n_keys ? vh[(size_t)key * D + d] : (_Float16)0.0f;
-            }
-            __builtin_memcpy(&v, e, 16);
-        }
-        ob[u] = v;
-    }
+// 16 bytes a lane from base + off to LDS bytes lds + 16·lane (base, lds uniform). As asm and not as the builtin: behind
+// the builtin the compiler makes the next LDS read wait for every load in flight (vmcnt 0), which it cannot tell apart
+// from the other buffer's; the asm writes no register, and the kernel waits for a stage's loads itself
+__device__ __forceinline__ void lds_load16(const void *base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
 }
 
-// OT: the output's type — f32, or f16 (rounded to nearest even: the value the f16 path's o-projection tile holds)
-template <typename OT>
-__global__ __launch_bounds__(256) void k_attn_causal(const float *q, const int4 *kvb, int n_blk, int n_q, int pos0,
-                                                     int n_head, int n_kv, float scale, OT *out) {
-    __shared__ __attribute__((aligned(16))) int4 s_kv[2][2][CB_CHUNKS];  // [buffer][half][chunk]
+// p − (float)h for the low (0) or high (1) half of h: one mixed-precision fma
+template <int HI> __device__ __forceinline__ float minus_half(float p, uint32_t h) {
+    float r;
+    if constexpr (HI) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(p));
+    else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(p));
+    return r;
+}
+
+// OT: the output's type — f32, or f16 (rounded to nearest even: the value the f16 path's o-projection tile holds).
+// POST: q holds the raw rows of the q projection; the head's RMS norm (weights qn) and RoPE are applied as they are read
+template <typename OT, bool POST>
+__global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float16 *kc, const _Float16 *vc, int n_q,
+                                                    int pos0, int n_head, int n_kv, int n_ctx, float scale,
+                                                    const float *qn, const float *rope, float eps, OT *out) {
+    __shared__ __attribute__((aligned(16))) int4 s_kv[2][CKS][CB_CHUNKS];  // [buffer][part][chunk]
+    __shared__ float s_ml[2 * CKS][2][CQ];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int g = lane >> 4, c = lane & 15;
-    const int n_qb = (n_q + CQ - 1) / CQ, half_grid = (n_qb + 1) / 2;
+    const int hf = lane >> 5, c = lane & 31;
+    const int n_qb = (n_q + CQ - 1) / CQ;
     const int kvh = blockIdx.x % n_kv, rank = blockIdx.x / n_kv;
-    const int qb = rank < half_grid ? n_qb - 1 - rank : rank - half_grid;
-    const int hh = wave & 1, kh = wave >> 1, h = 2 * kvh + hh;
+    const int half = (n_qb + 1) / 2, qb = rank < half ? n_qb - 1 - rank : rank - half;
+    const int hh = wave & 1, kp = wave >> 1, h = 2 * kvh + hh;
     const int q_first = CQ * qb, q_last = min(q_first + CQ - 1, n_q - 1);
     const int qi = min(q_first + c, n_q - 1), qpos = pos0 + qi;
-    const int nkb = (pos0 + q_last + 1 + CK - 1) / CK;  // key blocks the last query of the block sees
-    const int n_stage = (nkb + 1) / 2;
-    const int4 *src = kvb + (size_t)kvh * n_blk * CB_CHUNKS;
+    const int n_keys = pos0 + q_last + 1;                  // keys the last query of the block sees
+    const int nkb = (n_keys + CK - 1) / CK, n_stage = (nkb + CKS - 1) / CKS;
+    const int n_full = (pos0 + q_first + 1) / CK / CKS;     // stages whose keys every query sees
+    const _Float16 *kh = kc + (size_t)kvh * n_ctx * D, *vh = vc + (size_t)kvh * n_ctx * D;
 
-    // stage st → buffer: blocks 2st, 2st + 1 (clamped to the last: loaded, not used), 8 direct loads a wave
-    auto issue = [&](int st, int buf) {
+    // a stage's K or V → buffer st % 2: 4 direct loads a wave, each of the 4 waves 4 rows of 16 (keys past the last: the last)
+    const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int4 *)&s_kv[0][0][64 * wave];
+    const int lrow = 4 * wave + (lane >> 4), lc = lane & 15;
+    const uint32_t koff = 16 * (lc ^ (lrow & 15)), voff = 16 * (lc ^ (2 * (lrow & 7)));  // the same for row lrow + 16
+    auto issue = [&](int st, bool isv) {
+        const int s0 = CK * CKS * st;  // the stage's first key
+        const char *base = (const char *)(isv ? vh : kh) + (size_t)s0 * (2 * D);
+        const uint32_t off = isv ? voff : koff, last = 2 * D * (n_keys - 1 - s0) + off;  // the last key's
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int u = 64 * (wave + 4 * i);  // the wave's 64 chunks of the stage's 2048
-            const int blk = min(2 * st + (u >> 10), nkb - 1);
-            __builtin_amdgcn_global_load_lds((const void *)(src + (size_t)blk * CB_CHUNKS + (u & 1023) + lane),
-                                             (void __attribute__((address_space(3))) *)&s_kv[buf][u >> 10][u & 1023],
-                                             16, 0, 0);
-        }
+        for (int i = 0; i < 2 * CKS; i++)  // rows 16i + lrow of the stage: half a block
+            lds_load16(base, min(2 * D * (16 * i + lrow) + off, last),
+                       lds + (uint32_t)sizeof(int4) * (((st & 1) * CKS + i / 2) * CB_CHUNKS + (isv ? 512 : 0) + 256 * (i % 2)));
     };
-    issue(0, 0);
+    issue(0, false);
+    issue(0, true);
+    if (n_stage > 1) issue(1, false);
 
-    // q·scale as f16 pairs: B operand of step ks = dims 32ks + 8g … + 7 of query c
-    half8 qh[4], ql[4];
+    // q·scale as f16 pairs: B operand of step ks = dims 16ks + 8hf … + 7 of query c
+    half8 qh[8], ql[8];
     {
-        const float *qrow = q + ((size_t)qi * n_head + h) * D;
+        const float *qrow = q + ((size_t)qi * n_head + h) * D + 8 * hf;
+        float x[8][8];
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            const float4 a0 = *reinterpret_cast<const float4 *>(qrow + 32 * ks + 8 * g);
-            const float4 a1 = *reinterpret_cast<const float4 *>(qrow + 32 * ks + 8 * g + 4);
-            const float x[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        for (int ks = 0; ks < 8; ks++) {
+            const float4 a0 = *reinterpret_cast<const float4 *>(qrow + 16 * ks);
+            const float4 a1 = *reinterpret_cast<const float4 *>(qrow + 16 * ks + 4);
+            x[ks][0] = a0.x, x[ks][1] = a0.y, x[ks][2] = a0.z, x[ks][3] = a0.w;
+            x[ks][4] = a1.x, x[ks][5] = a1.y, x[ks][6] = a1.z, x[ks][7] = a1.w;
+        }
+        if constexpr (POST) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < 8; ks++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) ss = fmaf(x[ks][e], x[ks][e], ss);
+            const float inv = 1.0f / sqrtf(pair_sum<32>(ss) / (float)D + eps);
+            // the pairs (i, i + 64) are steps ks and ks + 4 of the same lane
+            const float *cs = rope + (size_t)qpos * D + 16 * hf;
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float2 t = *reinterpret_cast<const float2 *>(cs + 32 * ks + 2 * e);
+                    const float y0 = (x[ks][e] * inv) * qn[16 * ks + 8 * hf + e];
+                    const float y1 = (x[ks + 4][e] * inv) * qn[64 + 16 * ks + 8 * hf + e];
+                    x[ks][e] = y0 * t.x - y1 * t.y;
+                    x[ks + 4][e] = y0 * t.y + y1 * t.x;
+                }
+        }
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++)
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                const float qs = x[e] * scale;
+                float qs = x[ks][e] * scale;
+                // qs as one f32 value: the compiler otherwise rounds x·scale to f16 in two ways (from the product for
+                // qh, in one step for ql), which differ by an f16 ulp where the f32 rounding makes a tie
+                asm volatile("" : "+v"(qs));
                 const _Float16 hi = (_Float16)qs;
                 qh[ks][e] = hi;
                 ql[ks][e] = (_Float16)(qs - (float)hi);
             }
-        }
     }
-    f32x4 o[8];
+    // the lane's fragment slots in a block: K step ks (key c, dims 16ks + 8hf …); V tile t (16-lane group: dims
+    // 32t + 16(ℓ/16 % 2) …, keys 4hf + (ℓ%16)/4 of each 8-key group)
+    int ka[8], va[4];
 #pragma unroll
-    for (int t = 0; t < 8; t++) o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m = -3.0e38f, l = 0.0f;
+    for (int ks = 0; ks < 8; ks++) ka[ks] = 16 * c + ((2 * ks + hf) ^ (c & 15));
+    const int vrow = 4 * hf + ((lane & 15) >> 2);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+        va[t] = 16 * (512 + 16 * vrow + ((4 * t + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (2 * vrow))) + 8 * (lane & 1);
 
-    for (int st = 0; st < n_stage; st++) {
-        const int buf = st & 1;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads of stage st
-        __builtin_amdgcn_s_barrier();                       // everyone's; and stage st − 1 is read by all
+    f32x16 o[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[t][i] = 0.0f;
+    float nm = 3.0e38f, l = 0.0f;
+
+    auto scores = [&](f32x16 &s, int st) {
+        const int4 *blk = s_kv[st & 1][kp];
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) {
+            const half8 a = *reinterpret_cast<const half8 *>(blk + ka[ks]);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qh[ks], ks ? s : f32x16{}, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ql[ks], s, 0, 0, 0);
+        }
+    };
+    // stage st in buffer b: its scores are in s; the next stage's are computed into sn under the softmax's VALU work
+    auto step = [&](int st, int b, f32x16 &s, f32x16 &sn, auto mask) {
+        constexpr bool MASK = decltype(mask)::value;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads of K stage st + 1 and V stage st
+        __builtin_amdgcn_s_barrier();                       // everyone's; K stage st and V stage st − 1 are read by all
         asm volatile("" ::: "memory");
-        if (st + 1 < n_stage) issue(st + 1, buf ^ 1);
-        const int kb = 2 * st + kh;
-        if (kb >= nkb) continue;
-        const int4 *blk = s_kv[buf][kh];
-        f32x4 s[2];
+        if (st + 2 < n_stage) issue(st + 2, false);
+        if (st + 1 < n_stage) issue(st + 1, true);
+        const int k0 = CK * (CKS * st + kp);
+        float mx = -INFINITY;
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            s[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < 16; i++) {
+            if (MASK && k0 + 8 * (i >> 2) + 4 * hf + (i & 3) > qpos) s[i] = -INFINITY;  // keys after the query
+            mx = fmaxf(mx, s[i]);
+        }
+        mx = pair_max<32>(mx);
+        if (__builtin_amdgcn_ballot_w64(fmaf(mx, LOG2E, nm) > P_TOP)) {
+            const float to = fminf(nm, fmaf(-mx, LOG2E, P_SHIFT)), corr = __builtin_amdgcn_exp2f(to - nm);
+            nm = to;
+            l *= corr;
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                const half8 a = *reinterpret_cast<const half8 *>(blk + kb_kslot(16 * t + c, 4 * ks + g));
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[ks], s[t], 0, 0, 0);
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[ks], s[t], 0, 0, 0);
+            for (int t = 0; t < 4; t++) o[t] *= corr;
+        }
+        // the order pinned: behind each score MFMA of the next stage its share of this stage's softmax (left to itself
+        // the compiler issues the MFMAs back to back and the softmax behind them)
+        // (past the last stage: scores of what the buffer holds, not used)
+        const int4 *kb = s_kv[b ^ 1][kp];
+        const auto *vb = (const __attribute__((address_space(3))) char *)s_kv[b][kp];
+        // V tile t, step ss: slots 8hf … + 7 are keys 16ss + 4hf … + 3, then 16ss + 8 + 4hf … + 3 — the scores 8ss …
+        // that the lane holds
+        auto vread = [&](int t, int ss) {
+            const auto *p = vb + va[t] + 256 * 16 * ss;
+            const fp16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) fp16x4 *)p);
+            const fp16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) fp16x4 *)(p + 256 * 8));
+            half8 v;
+            __builtin_memcpy(&v, &lo, 8);
+            __builtin_memcpy((char *)&v + 8, &hi, 8);
+            return v;
+        };
+        uint32_t ph[8], pl[8];
+        half8 a[8], v[4];
+#pragma unroll
+        for (int ks = 0; ks < 3; ks++) a[ks] = *reinterpret_cast<const half8 *>(kb + ka[ks]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) {
+            sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks], qh[ks], ks ? sn : f32x16{}, 0, 0, 0);
+            if (ks + 3 < 8) a[ks + 3] = *reinterpret_cast<const half8 *>(kb + ka[ks + 3]);
+            else v[ks - 5] = vread(ks - 5, 0);
+            const float2_t p = {__builtin_amdgcn_exp2f(fmaf(s[2 * ks], LOG2E, nm)),
+                                __builtin_amdgcn_exp2f(fmaf(s[2 * ks + 1], LOG2E, nm))};  // masked: 2^(−inf) = 0
+            const half2_t hi = __builtin_convertvector(p, half2_t);
+            __builtin_memcpy(&ph[ks], &hi, 4);
+            asm volatile("" : "+v"(ph[ks]));  // holds the conversion here
+            __builtin_amdgcn_sched_barrier(0);
+            sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks], ql[ks], sn, 0, 0, 0);
+            l += p[0];
+            l += p[1];
+            const half2_t lo = __builtin_convertvector((float2_t{minus_half<0>(p[0], ph[ks]), minus_half<1>(p[1], ph[ks])}), half2_t);
+            __builtin_memcpy(&pl[ks], &lo, 4);
+            asm volatile("" : "+v"(pl[ks]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        v[3] = vread(3, 0);
+#pragma unroll
+        for (int ss = 0; ss < 2; ss++) {
+            half8 h8, l8;
+            __builtin_memcpy(&h8, &ph[4 * ss], 16);
+            __builtin_memcpy(&l8, &pl[4 * ss], 16);
+            half8 vn[4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[t], h8, o[t], 0, 0, 0);
+                if (ss == 0) vn[t] = vread(t, 1);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[t], l8, o[t], 0, 0, 0);
+                if (ss == 0) v[t] = vn[t];
             }
         }
-        // keys after the query (only in the block that holds the query block's positions) take no part
-        const bool diag = CK * kb + CK - 1 > pos0 + q_first;
-        float mx = m;
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                if (diag && CK * kb + 16 * t + 4 * g + r > qpos) s[t][r] = -INFINITY;
-                mx = fmaxf(mx, s[t][r]);
-            }
-        mx = pair_max<32>(pair_max<16>(mx));
-        const float corr = expf(m - mx);
-        float p[2][4], ps = 0.0f;
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                p[t][r] = expf(s[t][r] - mx);  // masked: e^(−inf) = 0
-                ps += p[t][r];
-            }
-        l = l * corr + pair_sum<32>(pair_sum<16>(ps));
-        m = mx;
-        if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {
-#pragma unroll
-            for (int t = 0; t < 8; t++) o[t] *= corr;
-        }
-        half8 ph, pl;
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float ps2 = p[t][r] * P_SCALE;
-                const _Float16 hi = (_Float16)ps2;
-                ph[4 * t + r] = hi;
-                pl[4 * t + r] = (_Float16)(ps2 - (float)hi);
-            }
-#pragma unroll
-        for (int t = 0; t < 8; t++) {
-            const half8 a = *reinterpret_cast<const half8 *>(blk + kb_vslot(16 * t + c, g));
-            o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ph, o[t], 0, 0, 0);
-            o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pl, o[t], 0, 0, 0);
-        }
+    };
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // K and V stage 0, K stage 1
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    f32x16 s0, s1;
+    scores(s0, 0);
+    int st = 0;
+    for (; st + 1 < n_full; st += 2) {
+        step(st, 0, s0, s1, std::false_type{});
+        step(st + 1, 1, s1, s0, std::false_type{});
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no LDS load in flight past this point
-    // merge the two key halves of each head through LDS (the stage buffers are free after this barrier)
-    __syncthreads();
-    float *s_o = reinterpret_cast<float *>(&s_kv[0][0][0]);  // [head][128 dims][16 queries] + [head][2][16]
-    float *s_ml = s_o + 2 * D * CQ;
-    if (kh == 1) {
-#pragma unroll
-        for (int t = 0; t < 8; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) s_o[(hh * D + 16 * t + 4 * g + r) * CQ + c] = o[t][r];
-        if (g == 0) {
-            s_ml[(hh * 2) * CQ + c] = m;
-            s_ml[(hh * 2 + 1) * CQ + c] = l;
-        }
+    for (; st < n_stage; st++) {
+        step(st, st & 1, s0, s1, std::true_type{});
+        s0 = s1;
     }
+    l = pair_sum<32>(l);
+    // merge the key parts of each head through LDS (the stage buffers, once every wave is done with them): every wave
+    // leaves its sums as its lanes hold them, then wave (head, part) finishes its share of the
+    // head's dims
     __syncthreads();
-    if (kh == 1 || q_first + c >= n_q) return;
-    const float m1 = s_ml[(hh * 2) * CQ + c], l1 = s_ml[(hh * 2 + 1) * CQ + c];
-    const float mm = fmaxf(m, m1), a0 = expf(m - mm), a1 = expf(m1 - mm);
-    const float inv = (1.0f / (l * a0 + l1 * a1)) * P_UNSCALE;
-    OT *orow = out + ((size_t)(q_first + c) * n_head + h) * D + 4 * g;
+    float *s_o = reinterpret_cast<float *>(&s_kv[0][0][0]);  // [wave][tile][register][lane]
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) s_o[((wave * 4 + t) * 16 + i) * 64 + lane] = o[t][i];
+    if (hf == 0) s_ml[wave][0][c] = nm, s_ml[wave][1][c] = l;
+    __syncthreads();
+    if (q_first + c >= n_q) return;
+    float w[CKS], lsum = 0.0f, top = 3.0e38f;
+#pragma unroll
+    for (int p = 0; p < CKS; p++) top = fminf(top, s_ml[2 * p + hh][0][c]);
+#pragma unroll
+    for (int p = 0; p < CKS; p++) {
+        w[p] = __builtin_amdgcn_exp2f(top - s_ml[2 * p + hh][0][c]);  // a part without keys: 2^(−3e38) = 0
+        lsum = fmaf(s_ml[2 * p + hh][1][c], w[p], lsum);
+    }
+    const float inv = 1.0f / lsum;
+    OT *orow = out + ((size_t)(q_first + c) * n_head + h) * D + 4 * hf;
+#pragma unroll
+    for (int u = 0; u < 16 / CKS; u++) {
+        const int t = kp * (4 / CKS) + (u >> 2), r = u & 3;
         float v[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) v[r] = (o[t][r] * a0 + s_o[(hh * D + 16 * t + 4 * g + r) * CQ + c] * a1) * inv;
-        if constexpr (sizeof(OT) == 4) {
-            *reinterpret_cast<float4 *>(orow + 16 * t) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-            const half4 hv = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-            *reinterpret_cast<half4 *>(orow + 16 * t) = hv;
+        for (int e = 0; e < 4; e++) {
+            v[e] = 0.0f;
+#pragma unroll
+            for (int p = 0; p < CKS; p++) v[e] = fmaf(s_o[(((2 * p + hh) * 4 + t) * 16 + 4 * r + e) * 64 + lane], w[p], v[e]);
+            v[e] *= inv;
         }
+        if constexpr (sizeof(OT) == 4) {
+            *reinterpret_cast<float4 *>(orow + 32 * t + 8 * r) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+            *reinterpret_cast<half4 *>(orow + 32 * t + 8 * r) =
+                half4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        }
+    }
+}
+
+// caches that are not 16-byte aligned, copied so that the direct loads can read them: [K, V][n_kv][n_keys][128]
+__global__ __launch_bounds__(256) void k_kv_align(const _Float16 *kc, const _Float16 *vc, int n_kv, int n_ctx,
+                                                  int n_keys, _Float16 *out) {
+    const size_t half = (size_t)n_kv * n_keys * D;
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < 2 * half; i += (size_t)gridDim.x * 256) {
+        const size_t j = i < half ? i : i - half, head = j / ((size_t)n_keys * D), r = j % ((size_t)n_keys * D);
+        out[i] = (i < half ? kc : vc)[head * n_ctx * D + r];
     }
 }
 
@@ -737,39 +840,33 @@ int launch_attn_decode(htr_device *dev, hipStream_t st, const float *q, const ui
     return htr_launched(dev, "k_attn_decode");
 }
 
-int launch_qk_norm_rope_rows(htr_device *dev, hipStream_t st, float *q, float *k, const float *v, const float *qn,
-                             const float *kn, const float *rope, int n_tok, int n_head, int n_kv, int pos0, int n_ctx,
-                             float eps, uint16_t *kc, uint16_t *vc) {
-    hipLaunchKernelGGL(k_qk_rows, dim3(n_tok, n_head + 2 * n_kv), dim3(64), 0, st, q, k, v, qn, kn, rope, n_head, n_kv,
-                       pos0, n_ctx, eps, (_Float16 *)kc, (_Float16 *)vc);
-    return htr_launched(dev, "k_qk_rows");
-}
-
-size_t attn_causal_block_bytes(int n_kv, int n_keys) {
-    return (size_t)n_kv * ((n_keys + CK - 1) / CK) * CB_CHUNKS * 16;
+int launch_kv_rows(htr_device *dev, hipStream_t st, const float *k, const float *v, const float *kn, const float *rope,
+                   int n_tok, int n_kv, int pos0, int n_ctx, float eps, uint16_t *kc, uint16_t *vc) {
+    const int n_rows = 2 * n_tok * n_kv;
+    hipLaunchKernelGGL(k_kv_rows, dim3((n_rows + 15) / 16), dim3(256), 0, st, k, v, kn, rope, n_rows, n_kv, pos0, n_ctx,
+                       eps, (_Float16 *)kc, (_Float16 *)vc);
+    return htr_launched(dev, "k_kv_rows");
 }
 
 int launch_attn_causal(htr_device *dev, hipStream_t st, const float *q, const uint16_t *kc, const uint16_t *vc,
-                       int n_q, int pos0, int n_head, int n_kv, int n_ctx, float scale, void *blocks, float *out,
-                       _Float16 *out16) {
+                       int n_q, int pos0, int n_head, int n_kv, int n_ctx, float scale, const CausalPost *post,
+                       float *out, _Float16 *out16) {
     if (n_head != 2 * n_kv) return htr_fail("causal attention: %d q heads on %d kv heads (groups of 2)", n_head, n_kv);
     if (n_q < 1 || pos0 < 0 || pos0 + n_q > n_ctx)
         return htr_fail("causal attention: %d queries from position %d in a %d-row cache", n_q, pos0, n_ctx);
     if (!out == !out16) return htr_fail("causal attention: one output, f32 or f16");
-    if (!blocks) return htr_fail("causal attention: no key-block buffer");
-    const int n_keys = pos0 + n_q, n_blk = (n_keys + CK - 1) / CK;
-    hipLaunchKernelGGL(k_kv_blocks, dim3(n_blk, n_kv), dim3(256), 0, st, (const _Float16 *)kc, (const _Float16 *)vc,
-                       n_ctx, n_keys, (int4 *)blocks);
-    HTR_TRY(htr_launched(dev, "k_kv_blocks"));
+    if (((uintptr_t)kc | (uintptr_t)vc) & 15) return htr_fail("causal attention: the caches must be 16-byte aligned");
     const dim3 grid(((n_q + CQ - 1) / CQ) * n_kv);
-    if (out) {
-        hipLaunchKernelGGL(k_attn_causal<float>, grid, dim3(256), 0, st, q, (const int4 *)blocks, n_blk, n_q, pos0,
-                           n_head, n_kv, scale, out);
-        return htr_launched(dev, "k_attn_causal");
-    }
-    hipLaunchKernelGGL(k_attn_causal<_Float16>, grid, dim3(256), 0, st, q, (const int4 *)blocks, n_blk, n_q, pos0,
-                       n_head, n_kv, scale, out16);
-    return htr_launched(dev, "k_attn_causal<f16>");
+    const CausalPost p = post ? *post : CausalPost{};
+#define HTR_CAUSAL(OT, POST, O)                                                                                        \
+    hipLaunchKernelGGL((k_attn_causal<OT, POST>), grid, dim3(CW), 0, st, q, (const _Float16 *)kc, (const _Float16 *)vc, \
+                       n_q, pos0, n_head, n_kv, n_ctx, scale, p.qn, p.rope, p.eps, O)
+    if (out && post) HTR_CAUSAL(float, true, out);
+    else if (out) HTR_CAUSAL(float, false, out);
+    else if (post) HTR_CAUSAL(_Float16, true, out16);
+    else HTR_CAUSAL(_Float16, false, out16);
+#undef HTR_CAUSAL
+    return htr_launched(dev, out ? "k_attn_causal" : "k_attn_causal<f16>");
 }
 
 // ---- the allocation-free decode attention ----------------------------------------------------------------------------
@@ -824,9 +921,20 @@ extern "C" int htr_causal_attention(htr_device *dev, const float *d_q, const uin
     if (!d_q || !d_k || !d_v || !d_out) return htr_fail("htr_causal_attention: null argument");
     if (n_q < 1 || pos0 < 0 || n_ctx < 1 || pos0 > n_ctx - n_q)
         return htr_fail("htr_causal_attention: %d queries from position %d in a %d-row cache", n_q, pos0, n_ctx);
-    void *blocks;
-    HTR_TRY(htr_scratch(dev, SCR_CAUSAL_BLOCKS, attn_causal_block_bytes(n_kv, pos0 + n_q), &blocks));
-    return launch_attn_causal(dev, dev->stream, d_q, d_k, d_v, n_q, pos0, n_head, n_kv, n_ctx, scale, blocks, d_out);
+    if (n_head != 2 * n_kv) return htr_fail("causal attention: %d q heads on %d kv heads (groups of 2)", n_head, n_kv);
+    if (((uintptr_t)d_k | (uintptr_t)d_v) & 15) {
+        const int n_keys = pos0 + n_q;
+        const size_t half = (size_t)n_kv * n_keys * D;
+        void *copy;
+        HTR_TRY(htr_scratch(dev, SCR_CAUSAL_KV, 2 * half * sizeof(_Float16), &copy));
+        hipLaunchKernelGGL(k_kv_align, dim3(dev->n_cu * 8), dim3(256), 0, dev->stream, (const _Float16 *)d_k,
+                           (const _Float16 *)d_v, n_kv, n_ctx, n_keys, (_Float16 *)copy);
+        HTR_TRY(htr_launched(dev, "k_kv_align"));
+        d_k = (const uint16_t *)copy;
+        d_v = d_k + half;
+        n_ctx = n_keys;
+    }
+    return launch_attn_causal(dev, dev->stream, d_q, d_k, d_v, n_q, pos0, n_head, n_kv, n_ctx, scale, nullptr, d_out);
 }
 
 extern "C" int htr_decode_attention(htr_device *dev, const float *d_q, const uint16_t *d_k, const uint16_t *d_v,

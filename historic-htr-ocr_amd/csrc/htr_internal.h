@@ -69,7 +69,7 @@ enum {
     SCR_CHOOSE_CNT = 1,
     SCR_ATTN_PART = 2,
     SCR_ATTN_CNT = 3,
-    SCR_CAUSAL_BLOCKS = 4,
+    SCR_CAUSAL_KV = 4,  // aligned copies of caches that are not
     SCR_GEMM_PART = 5,  // split-K products [split][M][N]
     SCR_HANDOVER = 6,   // htr_debug_handover's words
 };
@@ -153,17 +153,20 @@ struct AttnFuse {
 int launch_attn_decode(htr_device *dev, hipStream_t st, const float *q, const uint16_t *kc, const uint16_t *vc,
                        int n_head, int n_kv, int n_ctx, const int *pos_dev, int n_keys, float scale,
                        const AttnScratch &sc, float *out, const AttnFuse *fuse = nullptr, bool scale_after = false);
-// prefill pieces: per-head norm + rope + KV store over n_tok rows
-int launch_qk_norm_rope_rows(htr_device *dev, hipStream_t st, float *q, float *k, const float *v, const float *qn,
-                             const float *kn, const float *rope, int n_tok, int n_head, int n_kv, int pos0, int n_ctx,
-                             float eps, uint16_t *kc, uint16_t *vc);
-// the causal prefill attention: q [n_q][n_head·128] f32 (normed, roped), the head-major f16 caches [n_kv][n_ctx][128]
-// holding keys 0 … pos0 + n_q − 1; blocks: attn_causal_block_bytes(n_kv, pos0 + n_q) of device scratch (the key
-// blocks' copy); out [n_q][n_head·128] f32, or f16 into out16 (the f16 path's o-projection input) when out is NULL
-size_t attn_causal_block_bytes(int n_kv, int n_keys);
+// prefill pieces: the k heads' norm + rope and the K / V store over n_tok rows
+int launch_kv_rows(htr_device *dev, hipStream_t st, const float *k, const float *v, const float *kn, const float *rope,
+                   int n_tok, int n_kv, int pos0, int n_ctx, float eps, uint16_t *kc, uint16_t *vc);
+// the q heads' norm and rope done inside the causal attention (q then is the q projection's raw rows)
+struct CausalPost {
+    const float *qn, *rope;
+    float eps;
+};
+// the causal prefill attention: q [n_q][n_head·128] f32 (normed, roped, or raw with post), the head-major f16 caches
+// [n_kv][n_ctx][128] (16-byte aligned) holding keys 0 … pos0 + n_q − 1; out [n_q][n_head·128] f32, or f16 into out16
+// (the f16 path's o-projection input) when out is NULL
 int launch_attn_causal(htr_device *dev, hipStream_t st, const float *q, const uint16_t *kc, const uint16_t *vc,
-                       int n_q, int pos0, int n_head, int n_kv, int n_ctx, float scale, void *blocks, float *out,
-                       _Float16 *out16 = nullptr);
+                       int n_q, int pos0, int n_head, int n_kv, int n_ctx, float scale, const CausalPost *post,
+                       float *out, _Float16 *out16 = nullptr);
 
 // token choice (choose.hip)
 struct ChooseArgs {

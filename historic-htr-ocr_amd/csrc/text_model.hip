@@ -72,9 +72,6 @@ struct htr_session {
     hipGraphExec_t step_graph = nullptr;  // the CPU-choice step (no token choice)
     // the prefill's row buffers (ids, x, h, q, k, v, attention, g, u) for up to pre_cap rows, kept across calls
     void *pre = nullptr;
-    // the causal attention's key blocks (a copy of the cache's keys 0 … pos0 + n − 1 in its LDS layout), grown on demand
-    void *kvb = nullptr;
-    size_t kvb_bytes = 0;
     size_t pre_cap = 0;
     // the one-launch step (token_step.hip) for the 1024 / 2048 / 3072 decoder: its layer table, exchange words and
     // [seq, err] words; `fused` selects it for the decode step (fused_why: why it cannot be, when it cannot)
@@ -686,7 +683,7 @@ extern "C" int htr_session_free(htr_session *s) {
     if (s->step_graph) hipGraphExecDestroy(s->step_graph);
     for (void *p : {(void *)s->kc, (void *)s->vc, (void *)s->rope, (void *)s->x, (void *)s->qkv, (void *)s->attn,
                     (void *)s->g, (void *)s->logits, (void *)s->tok, (void *)s->state, (void *)s->asc.part,
-                    (void *)s->asc.counters, s->pre, s->kvb, (void *)s->h, (void *)s->u, (void *)s->tl, (void *)s->xw,
+                    (void *)s->asc.counters, s->pre, (void *)s->h, (void *)s->u, (void *)s->tl, (void *)s->xw,
                     (void *)s->tseq})
         if (p) htr_dev_free(dev, p);
     delete s;
@@ -896,14 +893,6 @@ extern "C" int htr_prefill(htr_session *s, const int32_t *ids, size_t n, float *
         rc = htr_dev_alloc(dev, n * per_row, HTR_MEM_WORK, &s->pre);
         if (rc == 0) s->pre_cap = n;
     }
-    const size_t kvb_need = attn_causal_block_bytes(c.n_kv, pos0 + l);
-    if (rc == 0 && kvb_need > s->kvb_bytes) {
-        if (s->kvb) htr_dev_free(dev, s->kvb);
-        s->kvb = nullptr;
-        s->kvb_bytes = 0;
-        rc = htr_dev_alloc(dev, kvb_need, HTR_MEM_WORK, &s->kvb);
-        if (rc == 0) s->kvb_bytes = kvb_need;
-    }
     uint32_t *d_tok = nullptr;
     float *x = nullptr, *h = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *a = nullptr, *g = nullptr,
           *u = nullptr;
@@ -933,10 +922,10 @@ extern "C" int htr_prefill(htr_session *s, const int32_t *ids, size_t n, float *
         uint16_t *kc = s->kc + li * s->kv_layer, *vc = s->vc + li * s->kv_layer;
         rc = launch_gemm_f16_qkv(dev, st, h16, l, ly.q, ly.k, ly.v, q, k, v);
         if (rc == 0)
-            rc = launch_qk_norm_rope_rows(dev, st, q, k, v, ly.q_norm, ly.k_norm, s->rope, l, c.n_head, c.n_kv, pos0,
-                                          s->kv_rows, c.eps, kc, vc);
+            rc = launch_kv_rows(dev, st, k, v, ly.k_norm, s->rope, l, c.n_kv, pos0, s->kv_rows, c.eps, kc, vc);
+        const CausalPost post = {ly.q_norm, s->rope, c.eps};
         if (rc == 0)
-            rc = launch_attn_causal(dev, st, q, kc, vc, l, pos0, c.n_head, c.n_kv, s->kv_rows, scale, s->kvb, nullptr,
+            rc = launch_attn_causal(dev, st, q, kc, vc, l, pos0, c.n_head, c.n_kv, s->kv_rows, scale, &post, nullptr,
                                     a16);
         if (rc == 0) rc = launch_gemm_f16_acc_norm(dev, st, a16, l, ly.o, x, ly.ffn_norm, c.eps, h16);
         if (rc == 0) rc = launch_gemm_f16(dev, st, GEMM_FFN, h16, l, ly.gate, ly.up, nullptr, g16, 1.0f);
@@ -955,9 +944,10 @@ extern "C" int htr_prefill(htr_session *s, const int32_t *ids, size_t n, float *
         if (rc == 0) rc = gemm(dev, st, h, ly.k, k, l, 0);
         if (rc == 0) rc = gemm(dev, st, h, ly.v, v, l, 0);
         if (rc == 0)
-            rc = launch_qk_norm_rope_rows(dev, st, q, k, v, ly.q_norm, ly.k_norm, s->rope, l, c.n_head, c.n_kv, pos0,
-                                          s->kv_rows, c.eps, kc, vc);
-        if (rc == 0) rc = launch_attn_causal(dev, st, q, kc, vc, l, pos0, c.n_head, c.n_kv, s->kv_rows, scale, s->kvb, a);
+            rc = launch_kv_rows(dev, st, k, v, ly.k_norm, s->rope, l, c.n_kv, pos0, s->kv_rows, c.eps, kc, vc);
+        const CausalPost post = {ly.q_norm, s->rope, c.eps};
+        if (rc == 0)
+            rc = launch_attn_causal(dev, st, q, kc, vc, l, pos0, c.n_head, c.n_kv, s->kv_rows, scale, &post, a);
         if (rc == 0) rc = gemm(dev, st, a, ly.o, x, l, 1);
         if (rc == 0) rc = launch_rms_norm(dev, st, x, ly.ffn_norm, h, l, d, c.eps);
         if (rc == 0) rc = gemm(dev, st, h, ly.gate, g, l, 0);
