@@ -324,6 +324,123 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const in
     }
 }
 
+// ---- the F32 path's K and V projections --------------------------------------------------------------------------------
+//
+// Y = X·Wᵀ with every output one chain of f32 fmas over k in order (matmul.wgsl:47-91), bit for bit: v_mfma_f32_16x16x4_f32
+// adds its four products one after another, each rounded. K and V are rounded to f16 into the cache, where a last-bit
+// difference of the f32 sum can move a value by an f16 ulp, which then stays in every later layer: with these two products
+// in the reference's order the logits of a 1023-token prompt through 28 layers are 4.5e-5 from the f32 oracle's, with the
+// exact block sums of k_gemm_q8_0 (which no order of f32 sums equals) 1.15e-4.
+// A workgroup owns 32 × 64 outputs of one of the two matrices (grid z), 4 waves of 16 × 32; K in stages of two q8_0
+// blocks, double-buffered in LDS as f32, their loads two stages ahead. A row's 32 values lie by k mod 4, then k / 4, so a lane's operands of the 8 MFMAs (k = 4s
+// + its quarter) are two 16-byte chunks, placed at chunk ^ (row/2 % 8). Bound: the
+// stages' latency at prompt sizes (333 × 2 · 1024 × 1024 28.7 µs a launch, 49 TFLOP/s; one block a stage 33.5 µs).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+struct KvGemm {
+    const int8_t *q[2];
+    const _Float16 *d[2];
+    float *y[2];
+};
+
+__global__ __launch_bounds__(256) void k_gemm_q8_0_chain(const float *x, const KvGemm w, int m, int n, int k) {
+    constexpr int KB = 2;  // blocks a stage; a last odd one is followed by zeros (0·0 + c = c)
+    __shared__ __attribute__((aligned(16))) float s_a[2][KB][32 * 32], s_b[2][KB][64 * 32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1, row0 = blockIdx.y * 32, col0 = blockIdx.x * 64, nb = k / 32;
+    // staging: k 8·lq … + 7 of both blocks of W row lr, and of one block (the thread's half) of X row lr % 32
+    const int lr = tid >> 2, lq = tid & 3, ab = tid >> 7, ar = lr & 31;
+    const float *xr = x + (size_t)min(row0 + ar, m - 1) * k + 8 * lq;
+    const int8_t *wq = w.q[blockIdx.z] + (size_t)(col0 + lr) * k + 8 * lq;
+    const _Float16 *wd = w.d[blockIdx.z] + (size_t)(col0 + lr) * nb;
+    struct Regs {
+        float4 a0, a1;
+        int2 q[KB];
+        _Float16 d[KB];
+    };
+    auto gload = [&](Regs &r, int st) {
+        const float4 *xs = reinterpret_cast<const float4 *>(xr + 32 * min(KB * st + ab, nb - 1));
+        r.a0 = xs[0];
+        r.a1 = xs[1];
+#pragma unroll
+        for (int i = 0; i < KB; i++) {
+            const int kb = min(KB * st + i, nb - 1);
+            r.q[i] = *reinterpret_cast<const int2 *>(wq + 32 * kb);
+            r.d[i] = wd[kb];
+        }
+    };
+    // the float slot of (row r, quarter k mod 4 = t, k / 4 = 2·lq): the pair (2·lq, 2·lq + 1) is contiguous
+    auto slot = [](int r, int t, int l) { return 32 * r + 4 * ((2 * t + (l >> 1)) ^ ((r >> 1) & 7)) + 2 * (l & 1); };
+    auto lstore = [&](const Regs &r, int st) {
+        const float a[8] = {r.a0.x, r.a0.y, r.a0.z, r.a0.w, r.a1.x, r.a1.y, r.a1.z, r.a1.w};
+        const bool in = KB * st + ab < nb;
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            *reinterpret_cast<float2 *>(&s_a[st & 1][ab][slot(ar, t, lq)]) = in ? make_float2(a[t], a[4 + t]) : make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int i = 0; i < KB; i++) {
+            const float d = KB * st + i < nb ? (float)r.d[i] : 0.0f;
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+                *reinterpret_cast<float2 *>(&s_b[st & 1][i][slot(lr, t, lq)]) =
+                    make_float2((float)q_byte(r.q[i], t) * d, (float)q_byte(r.q[i], 4 + t) * d);
+        }
+    };
+    f32x4 c[2] = {f32x4{}, f32x4{}};
+    const int fa = 16 * wm + (lane & 15), fb = 32 * wn + (lane & 15), t = lane >> 4;
+    auto frag = [&](const float *s, int r, float (&f)[8]) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float4 v = *reinterpret_cast<const float4 *>(s + slot(r, t, 2 * h));
+            f[4 * h] = v.x, f[4 * h + 1] = v.y, f[4 * h + 2] = v.z, f[4 * h + 3] = v.w;
+        }
+    };
+    // LDS accesses done at the barrier, the next stages' register loads left in flight
+    auto lds_barrier = [] {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    const int nst = (nb + KB - 1) / KB;
+    Regs ring[2];
+    gload(ring[0], 0);
+    gload(ring[1], 1);
+    lstore(ring[0], 0);
+    gload(ring[0], 2);
+    lds_barrier();
+    for (int s0 = 0; s0 < nst; s0 += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int st = s0 + u;
+            if (st >= nst) break;
+            float a[KB][8], b[KB][2][8];
+#pragma unroll
+            for (int i = 0; i < KB; i++) {
+                frag(s_a[u][i], fa, a[i]);
+                frag(s_b[u][i], fb, b[i][0]);
+                frag(s_b[u][i], fb + 16, b[i][1]);
+            }
+#pragma unroll
+            for (int i = 0; i < KB; i++)
+#pragma unroll
+                for (int s = 0; s < 8; s++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) c[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][s], b[i][j][s], c[j], 0, 0, 0);
+            if (st + 1 < nst) lstore(ring[u ^ 1], st + 1);
+            gload(ring[u ^ 1], st + 3);
+            lds_barrier();
+        }
+    }
+    // lane ℓ, register r: row 4(ℓ/16) + r, column ℓ%16
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int row = row0 + 16 * wm + 4 * t + r;
+            if (row < m) w.y[blockIdx.z][(size_t)row * n + col0 + 32 * wn + 16 * j + (lane & 15)] = c[j][r];
+        }
+}
+
 // the f16 plane of a q8_0 weight: h = f16(q · d) (round to nearest even), 8 values a thread
 __global__ __launch_bounds__(256) void k_q8_to_f16(const int8_t *q, const _Float16 *d, _Float16 *h, size_t n8,
                                                     int cols) {
@@ -383,6 +500,17 @@ int launch_gemm_q8_0_f32(htr_device *dev, hipStream_t st, const float *x, const 
 int launch_gemm_q8_0_r16(htr_device *dev, hipStream_t st, const float *x, const htr_weight *w, float *y, int m,
                          int acc) {
     return gemm_q8<false>(dev, st, x, w, y, m, acc);
+}
+
+int launch_gemm_q8_0_kv(htr_device *dev, hipStream_t st, const float *x, const htr_weight *wk, const htr_weight *wv,
+                        float *k, float *v, int m) {
+    const int n = (int)wk->rows, cols = (int)wk->cols;
+    if (!wk->q || !wv->q || wv->rows != wk->rows || wv->cols != wk->cols || n % 64 || cols % 32)
+        return htr_fail("gemm_kv: K [%zu x %zu], V [%zu x %zu]: equal, rows a multiple of 64", wk->rows, wk->cols, wv->rows,
+                        wv->cols);
+    const KvGemm w = {{wk->q, wv->q}, {wk->d, wv->d}, {k, v}};
+    hipLaunchKernelGGL(k_gemm_q8_0_chain, dim3(n / 64, (m + 31) / 32, 2), dim3(256), 0, st, x, w, m, n, cols);
+    return htr_launched(dev, "k_gemm_q8_0_chain");
 }
 
 int launch_rms_norm(htr_device *dev, hipStream_t st, const float *x, const float *w, float *y, int rows, int dim,

@@ -72,6 +72,7 @@ enum {
     SCR_CAUSAL_KV = 4,  // aligned copies of caches that are not
     SCR_GEMM_PART = 5,  // split-K products [split][M][N]
     SCR_HANDOVER = 6,   // htr_debug_handover's words
+    SCR_VISION_PART = 7,  // the vision attention's sums of tiles cut along their keys
 };
 // the device's scratch buffer `slot` with at least `bytes` bytes (a larger one replaces it: the tickets' and best
 // keys' slots zero-filled, the others as htr_dev_alloc fills)
@@ -198,6 +199,9 @@ int launch_choose(htr_device *dev, hipStream_t st, const ChooseArgs &a);
 // f16 at the tiles (the f16 compute path, any shape); rms_norm rows; swiglu; a weight's f16 plane made on the device
 int launch_gemm_q8_0_f32(htr_device *dev, hipStream_t st, const float *x, const htr_weight *w, float *y, int m,
                          int acc);
+// K = X·Wkᵀ, V = X·Wvᵀ in f32, each output one fma chain over k in order (the F32 path's cache rows)
+int launch_gemm_q8_0_kv(htr_device *dev, hipStream_t st, const float *x, const htr_weight *wk, const htr_weight *wv,
+                        float *k, float *v, int m);
 int launch_gemm_q8_0_r16(htr_device *dev, hipStream_t st, const float *x, const htr_weight *w, float *y, int m,
                          int acc);
 int weight_attach_f16(htr_device *dev, hipStream_t st, htr_weight *w);

@@ -941,8 +941,12 @@ extern "C" int htr_prefill(htr_session *s, const int32_t *ids, size_t n, float *
         uint16_t *kc = s->kc + li * s->kv_layer, *vc = s->vc + li * s->kv_layer;
         rc = launch_rms_norm(dev, st, x, ly.attn_norm, h, l, d, c.eps);
         if (rc == 0) rc = gemm(dev, st, h, ly.q, q, l, 0);
-        if (rc == 0) rc = gemm(dev, st, h, ly.k, k, l, 0);
-        if (rc == 0) rc = gemm(dev, st, h, ly.v, v, l, 0);
+        if (rc == 0 && m->compute == HTR_COMPUTE_F32) {
+            rc = launch_gemm_q8_0_kv(dev, st, h, ly.k, ly.v, k, v, l);
+        } else {
+            if (rc == 0) rc = gemm(dev, st, h, ly.k, k, l, 0);
+            if (rc == 0) rc = gemm(dev, st, h, ly.v, v, l, 0);
+        }
         if (rc == 0)
             rc = launch_kv_rows(dev, st, k, v, ly.k_norm, s->rope, l, c.n_kv, pos0, s->kv_rows, c.eps, kc, vc);
         const CausalPost post = {ly.q_norm, s->rope, c.eps};

@@ -297,6 +297,41 @@ def test_matmul_q8_0_f32_path_keeps_infinities_and_nans(dev):
     w.free()
 
 
+# one block; an odd block count; row counts around the tile of 32; the decoder's width
+@pytest.mark.parametrize("n_tok,dim,n_kv", [(1, 32, 1), (31, 96, 2), (33, 160, 1), (65, 1024, 2)])
+def test_f32_prefill_values_are_the_reference_fma_chain(dev, n_tok, dim, n_kv):
+    """the F32 path's V rows in the cache, bit for bit: every output one chain of f32 fmas over k in order, rounded to
+    f16. The embedding is ±1 and 1 + eps is 1 in f32, so the projection's input is ± the norm's weights on any machine"""
+    import oracle as orc
+
+    n_head, n_ff, n_vocab, eps = 2 * n_kv, 64, 300, 1e-9
+    sign = np.where(htr.synth_normal(dim, n_vocab * dim) < 0, -1, 1).astype(np.int8).reshape(n_vocab, dim // 32, 32)
+    emb = np.empty((n_vocab, dim // 32, 34), np.uint8)
+    emb[:, :, :2] = np.array([2.0 ** -6], np.float16).view(np.uint8)
+    emb[:, :, 2:] = (64 * sign).view(np.uint8)
+    qd, kvd = n_head * 128, n_kv * 128
+    ly = {n: htr.synth_q8_0(i + dim, r, c) for i, (n, r, c) in enumerate((
+        ("q", qd, dim), ("k", kvd, dim), ("v", kvd, dim), ("o", dim, qd), ("gate", n_ff, dim), ("up", n_ff, dim),
+        ("down", dim, n_ff)))}
+    ly.update(attn_norm=htr.synth_normal(1, dim), ffn_norm=htr.synth_normal(2, dim), q_norm=htr.synth_normal(3, 128),
+              k_norm=htr.synth_normal(4, 128))
+    cfg = htr.TextConfig(n_layer=1, dim=dim, n_head=n_head, n_kv=n_kv, d_head=128, n_ff=n_ff, n_vocab=n_vocab,
+                         n_ctx_train=4096, eps=eps, rope_base=1e6)
+    ids = np.random.default_rng(n_tok).integers(0, n_vocab, n_tok).astype(np.int32)
+    keep, dev.compute = dev.compute, htr.COMPUTE_F32
+    try:
+        m = htr.TextModel(dev, cfg, emb.reshape(-1), htr.synth_normal(5, dim), [ly])
+    finally:
+        dev.compute = keep
+    s = m.session(n_tok)
+    s.prefill(ids)
+    got = s.kv_rows(0, 0, n_tok)[1]
+    h = sign[ids].reshape(n_tok, dim).astype(np.float32) * ly["attn_norm"]
+    assert np.array_equal(got, orc.f16_bits(orc.matmul_q8_0(h, ly["v"], kvd).ravel()).reshape(n_tok, kvd))
+    s.free()
+    m.free()
+
+
 def test_compute_path_setting(dev):
     keep = dev.compute
     assert keep in (htr.COMPUTE_F32, htr.COMPUTE_F16)
