@@ -498,13 +498,6 @@ typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef __fp16 fp16x4 __attribute__((ext_vector_type(4)));
 
-// 16 bytes a lane from base + off to LDS bytes lds + 16·lane (base, lds uniform). As asm and not as the builtin: behind
-// the builtin the compiler makes the next LDS read wait for every load in flight (vmcnt 0), which it cannot tell apart
-// from the other buffer's; the asm writes no register, and the kernel waits for a stage's loads itself
-__device__ __forceinline__ void lds_load16(const void *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
-}
-
 // p − (float)h for the low (0) or high (1) half of h: one mixed-precision fma
 template <int HI> __device__ __forceinline__ float minus_half(float p, uint32_t h) {
     float r;
@@ -587,10 +580,7 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
         for (int ks = 0; ks < 8; ks++)
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                float qs = x[ks][e] * scale;
-                // qs as one f32 value: the compiler otherwise rounds x·scale to f16 in two ways (from the product for
-                // qh, in one step for ql), which differ by an f16 ulp where the f32 rounding makes a tie
-                asm volatile("" : "+v"(qs));
+                const float qs = x[ks][e] * scale;
                 const _Float16 hi = (_Float16)qs;
                 qh[ks][e] = hi;
                 ql[ks][e] = (_Float16)(qs - (float)hi);

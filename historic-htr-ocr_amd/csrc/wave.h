@@ -111,3 +111,10 @@ template <int N> __device__ __forceinline__ float wave_sum_rows(float (&v)[N], i
     halve<N, 32, S>(v, lane);
     return group_sum<(32 >> S)>(v[0], lane);
 }
+
+// 16 bytes a lane from base + off to LDS bytes lds + 16·lane (base, lds uniform). As asm and not as the builtin: behind
+// the builtin the compiler makes the next LDS read wait for every load in flight (vmcnt 0), which it cannot tell apart
+// from the other buffer's; the asm writes no register, and the kernel waits for a stage's loads itself
+__device__ __forceinline__ void lds_load16(const void *base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}

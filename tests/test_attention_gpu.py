@@ -179,7 +179,7 @@ def test_causal_attention_block_edges(dev, n_q, pos0, n_kv, scale_q, off):
         raw = kv_head_major(a, n_kv).view(np.uint16).ravel()
         bufs.append(dev.upload(np.concatenate([np.zeros(off, np.uint16), raw, np.zeros(8 - off, np.uint16)])))
     out = dev.alloc(n_q * n_head * 128 * 4)
-    sc = float(np.float32(1 / np.sqrt(128)))
+    sc = 0.125  # exact in f32: q·scale is the same value however it is rounded to f16
     qb = dev.upload(q)
     rc = htr.lib().htr_causal_attention(dev.h, qb.ptr, bufs[0].ptr + 2 * off, bufs[1].ptr + 2 * off, n_q, pos0, n_head,
                                         n_kv, n_keys, sc, out.ptr)
@@ -187,5 +187,5 @@ def test_causal_attention_block_edges(dev, n_q, pos0, n_kv, scale_q, off):
     got = out.download(np.float32).reshape(n_q, n_head * 128)
     for t in range(n_q):
         row = orc.attn_f64(q[t * n_head * 128:(t + 1) * n_head * 128], k, v, n_kv * 128, pos0 + t + 1, n_head, n_kv,
-                           1 / np.sqrt(128))
+                           sc)
         assert rel_l2(got[t], row) < 1e-5 * max(1.0, scale_q / 4), t
