@@ -155,45 +155,42 @@ __global__ __launch_bounds__(VW) void k_heads_f16(const float *K, const float *V
 // MFMAs 32x32x16: lane ℓ = 32h + c then holds query c's scores of keys 8(i / 4) + 4h + i % 4 (i < 16), the other 16
 // in lane ℓ ^ 32. Oᵀ (64 dims × 32 queries) += Vᵀ·Pᵀ is 4 more, lane ℓ accumulating dims 32t + 8(i / 4) + 4h + i % 4
 // of query c, so the rescale by the query's corr stays in the lane.
-// The 4 waves of a workgroup (128·QG queries) share the key blocks: stages of AST blocks are copied from memory to LDS
-// (coalesced 16-byte loads, the next stage's in flight while the current one is in use) and each wave reads its
-// fragments from there. grid: ⌈n / (128·QG)⌉ · H workgroups, numbered so that the workgroups of one head run on one
-// XCD.
+// The 4 waves of a workgroup (128·QG queries) share the key blocks: stages of AST blocks are copied from memory to LDS by
+// direct loads, the next stage's in flight while the current one is in use, and each wave reads its fragments from there.
+// Work: a page makes n_head · ⌈n / (128·QG)⌉ tiles, a workgroup is one of two on every CU (`workers` a group), and an
+// uneven last round would cost as much as a full one. So each worker takes whole tiles while the rounds are full, and the
+// tiles that are left are cut along their keys into equal shares, one a worker, whose sums go to memory and are joined by
+// k_attn_vision_merge. The workers of a group (with H a multiple of 8: an XCD, workgroup b runs on XCD b % 8) share its
+// heads, so a head's keys stay in one XCD's L2.
 constexpr int FQ = 32, FB = 32, FWAVES = VW / 64, AST = 2;
+// p = 2^(s·log2 e + nm), nm = 10 − log2 e · (the max when it was last moved): nm moves, and O and l are rescaled, only
+// when some p would pass 2^15 (f16 holds 65504), so most blocks skip the rescale; nm is the only state, its rounding
+// cancels between p, l and O
+constexpr float P_SHIFT = 10.0f, P_TOP = 15.0f, LOG2E = 1.4426950408889634f;
+constexpr int RING = 3;      // stages in LDS: the one in use, the next one (its first K block), one loading
+constexpr int CUT_COST = 8;  // stages that a cut has to save: the partial sums' way through memory and the merge's launch
+
+struct VSplit {
+    int groups, workers;      // groups of heads; workers a group
+    int tiles, full;          // tiles a group; the first `full` of them are taken whole
+    int n_qt, n_stage;        // tiles a head; stages of AST key blocks
+    __host__ __device__ int first(int i) const {  // the first of worker i's stages of the tiles that are cut
+        return (int)((long long)(tiles - full) * n_stage * i / workers);
+    }
+};
+// a worker's sums of a part of a tile: [wave][query group][dim tile][16] registers, then nm and l, × 64 lanes
+template <int QG> constexpr int PART = FWAVES * QG * 34 * 64;
 
 // QG groups of 32 queries a wave: the groups share every K / V fragment read from LDS and give the wave QG
 // independent chains (Sᵀ MFMAs → max → exp → P·V) to interleave
 template <int QG>
 __global__ __launch_bounds__(VW) void k_attn_vision(const float *Q, const _Float16 *KV, _Float16 *O, int n_tok,
-                                                    int n_head, int n_blk, int n_qt, float scale, const float *cs,
-                                                    int px, int max_pos) {
-    __shared__ __attribute__((aligned(16))) half8 s_kv[2][AST * KVB / 16];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hf = lane >> 5, c = lane & 31;
-    // workgroup b runs on XCD b % 8: with H a multiple of 8, XCD x takes heads x·H/8 … (x + 1)·H/8 − 1
-    int h, qt;
-    if (n_head % 8 == 0) {
-        const int i = blockIdx.x / 8;
-        h = (blockIdx.x % 8) * (n_head / 8) + i / n_qt;
-        qt = i % n_qt;
-    } else {
-        h = blockIdx.x / n_qt;
-        qt = blockIdx.x % n_qt;
-    }
-    const int row = n_head * 64, q0 = (qt * FWAVES + wave) * FQ * QG;
-    half8 qf[QG][4];  // B operand of step ks: q16[query c][dims 16ks + 8h … + 7], q turned by rope2d first
-#pragma unroll
-    for (int g = 0; g < QG; g++) {
-        const int qi = min(q0 + FQ * g + c, n_tok - 1);
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            const float4 *src = reinterpret_cast<const float4 *>(Q + (size_t)qi * row + h * 64 + 16 * ks + 8 * hf);
-            const float4 x0 = src[0], x1 = src[1];
-            float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-            rope8(x, cs, qi, px, max_pos, 16 * ks + 8 * hf);
-#pragma unroll
-            for (int e = 0; e < 8; e++) qf[g][ks][e] = (_Float16)(x[e] * scale);
-        }
-    }
+                                                    int n_head, int n_blk, VSplit sp, float scale, const float *cs,
+                                                    int px, int max_pos, float *part) {
+    __shared__ __attribute__((aligned(16))) half8 s_kv[RING][AST * KVB / 16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hf = lane >> 5, c = lane & 31;
+    const int grp = blockIdx.x % sp.groups, wk = blockIdx.x / sp.groups, row = n_head * 64;
+    const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) half8 *)&s_kv[0][64 * wave];
     // the lane's fragment chunks within a block: K step ks (key c, dims 16ks + 8h …), Vᵀ tile t step st (dim 32t + c,
     // slots 16st + 8h …)
     int kc[4], vc[4];
@@ -203,131 +200,208 @@ __global__ __launch_bounds__(VW) void k_attn_vision(const float *Q, const _Float
     for (int t = 0; t < 2; t++)
 #pragma unroll
         for (int st = 0; st < 2; st++) vc[2 * t + st] = kv_vchunk(32 * t + c, 2 * st + hf);
-    // stage copies: AST blocks of 512 chunks, 2·AST chunks a thread (blocks past the last repeat it: in bounds)
-    const half8 *gkv = reinterpret_cast<const half8 *>(KV) + (size_t)h * n_blk * (KVB / 16);
-    half8 stg[2 * AST];
-    auto gload = [&](int stage) {
+    // stages 0 … n_full − 1 hold keys < n_tok only
+    const int n_full = n_tok / (AST * FB);
+
+    // stages st0 … st1 − 1 of a tile; slot: where the sums go, −1: the tile is whole
+    auto run = [&](int tile, int st0, int st1, int slot) {
+        const int h = grp * (n_head / sp.groups) + tile / sp.n_qt, q0 = ((tile % sp.n_qt) * FWAVES + wave) * FQ * QG;
+        const char *gkv = (const char *)KV + (size_t)h * n_blk * KVB;
+        // a stage is 16 KB: 4 direct loads a wave (blocks past the last repeat it: in bounds)
+        auto issue = [&](int st) {
 #pragma unroll
-        for (int i = 0; i < 2 * AST; i++) {
-            const int blk = min(stage * AST + i / 2, n_blk - 1);
-            stg[i] = gkv[(size_t)blk * (KVB / 16) + (i % 2) * VW + tid];
-        }
-    };
-    auto lstore = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < 2 * AST; i++) s_kv[buf][(i / 2) * (KVB / 16) + (i % 2) * VW + tid] = stg[i];
-    };
-    f32x16 o[QG][2];
-    float m[QG], l[QG];
-#pragma unroll
-    for (int g = 0; g < QG; g++) {
-        m[g] = -3.0e38f;
-        l[g] = 0.0f;
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) o[g][t][i] = 0.0f;
-    }
-    // one key block at k0 from LDS; MASK: the block holds keys ≥ n_tok (the last one only), which take no part in
-    // the max and get p = 0. A rescale by corr = 1 is skipped (x·1 = x).
-    auto block = [&](const half8 *sb, int k0, auto mask) {
-        constexpr bool MASK = decltype(mask)::value;
-        half8 fk[4], fv[4];
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) fk[ks] = sb[kc[ks]];
-#pragma unroll
-        for (int i = 0; i < 4; i++) fv[i] = sb[vc[i]];
-        f32x16 s[QG];
+            for (int i = 0; i < 2 * AST; i++)
+                lds_load16(gkv + (size_t)min(st * AST + i / 2, n_blk - 1) * KVB + (i % 2) * (VW * 16), 16 * tid,
+                           lds + (st % RING) * (AST * KVB) + i * (VW * 16));
+        };
+        issue(st0);
+        if (st0 + 1 < st1) issue(st0 + 1);
+        half8 qf[QG][4];  // B operand of step ks: q16[query c][dims 16ks + 8h … + 7], q turned by rope2d first
 #pragma unroll
         for (int g = 0; g < QG; g++) {
+            const int qi = min(q0 + FQ * g + c, n_tok - 1);
 #pragma unroll
-            for (int i = 0; i < 16; i++) s[g][i] = 0.0f;
+            for (int ks = 0; ks < 4; ks++) {
+                const float4 *src = reinterpret_cast<const float4 *>(Q + (size_t)qi * row + h * 64 + 16 * ks + 8 * hf);
+                const float4 x0 = src[0], x1 = src[1];
+                float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+                rope8(x, cs, qi, px, max_pos, 16 * ks + 8 * hf);
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) s[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fk[ks], qf[g][ks], s[g], 0, 0, 0);
-        }
-        half8 pb[QG][2];
-#pragma unroll
-        for (int g = 0; g < QG; g++) {
-            float mx = m[g];
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-                if (!MASK || k0 + 8 * (i >> 2) + 4 * hf + (i & 3) < n_tok) mx = fmaxf(mx, s[g][i]);
-            mx = pair_max<32>(mx);
-            // e^(s − mx) = 2^(s·log2 e − mx·log2 e): one fma and v_exp_f32 a score; P rounded to f16 in pairs
-            // (v_cvt_pk_f16_f32, round to nearest even) and summed as f32 by v_dot2 against (1, 1)
-            constexpr float LOG2E = 1.4426950408889634f;
-            const float corr = __builtin_amdgcn_exp2f((m[g] - mx) * LOG2E), nml = -mx * LOG2E;
-            if (__builtin_amdgcn_ballot_w64(corr != 1.0f)) {
-#pragma unroll
-                for (int t = 0; t < 2; t++) o[g][t] *= corr;
+                for (int e = 0; e < 8; e++) qf[g][ks][e] = (_Float16)(x[e] * scale);
             }
-            float ps = 0.0f;
+        }
+        f32x16 o[QG][2];
+        float nm[QG], l[QG];
 #pragma unroll
-            for (int i = 0; i < 16; i += 2) {
-                float2_t e = {__builtin_amdgcn_exp2f(fmaf(s[g][i], LOG2E, nml)),
-                              __builtin_amdgcn_exp2f(fmaf(s[g][i + 1], LOG2E, nml))};
-                if (MASK) {
-                    if (k0 + 8 * (i >> 2) + 4 * hf + (i & 3) >= n_tok) e[0] = 0.0f;
-                    if (k0 + 8 * (i >> 2) + 4 * hf + (i & 3) + 1 >= n_tok) e[1] = 0.0f;
+        for (int g = 0; g < QG; g++) {
+            nm[g] = 3.0e38f;
+            l[g] = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) o[g][t][i] = 0.0f;
+        }
+        // the two groups take turns: while the VALU does group X's softmax of block j, the matrix pipe does group Y's next
+        // scores and its P·V of the block before. Phase 0: X = 0, Y = 1 with the scores of block j, P·V of j − 1, and K of
+        // block j + 1 read behind them; phase 1: X = 1, Y = 0 with the scores of block j + 1, V of block j read, then P·V
+        // of j. The order is pinned: behind each MFMA two scores' share of the softmax
+        f32x16 sc[QG];
+        half8 kf[4], vf[4] = {};
+        uint32_t pb[QG][8] = {};
+        auto kread = [&](const half8 *blk, int ks) { kf[ks] = blk[kc[ks]]; };
+        auto pv = [&](int g, int i) {
+            const int t = i & 1, st = i >> 1;
+            half8 p;
+            __builtin_memcpy(&p, &pb[g][4 * st], 16);
+            o[g][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[2 * t + st], p, o[g][t], 0, 0, 0);
+        };
+        auto score = [&](int g, int ks) {
+            sc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[g][ks], ks ? sc[g] : f32x16{}, 0, 0, 0);
+        };
+        // blk: block j; nxt: block j + 1 (past the last one: whatever the buffer holds; its scores are not used); k0: the
+        // block's first key; MASK: keys ≥ n_tok score −inf
+        auto step = [&](const half8 *blk, const half8 *nxt, int k0, auto mask) {
+            constexpr bool MASK = decltype(mask)::value;
+#pragma unroll
+            for (int X = 0; X < QG; X++) {
+                const int Y = X ^ 1;
+                float mx = -INFINITY;
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    if (MASK && k0 + 8 * (i >> 2) + 4 * hf + (i & 3) >= n_tok) sc[X][i] = -INFINITY;
+                    mx = fmaxf(mx, sc[X][i]);
                 }
-                const half2_t p2 = __builtin_convertvector(e, half2_t);
-                pb[g][i >> 3][i & 7] = p2[0];
-                pb[g][i >> 3][(i & 7) + 1] = p2[1];
-                ps = __builtin_amdgcn_fdot2(p2, half2_t{(_Float16)1.0f, (_Float16)1.0f}, ps, false);
+                mx = pair_max<32>(mx);
+                if (__builtin_amdgcn_ballot_w64(fmaf(mx, LOG2E, nm[X]) > P_TOP)) {
+                    const float to = fminf(nm[X], fmaf(-mx, LOG2E, P_SHIFT)), corr = __builtin_amdgcn_exp2f(to - nm[X]);
+                    nm[X] = to;
+                    l[X] *= corr;
+#pragma unroll
+                    for (int t = 0; t < 2; t++) o[X][t] *= corr;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    if (i < 4) score(Y, i);
+                    else pv(Y, i - 4);
+                    if (X == 0 && i >= 4) kread(nxt, i - 4);
+                    if (X == 1 && i < 4) vf[i] = blk[vc[i]];
+                    // P rounded to f16 in pairs (v_cvt_pk_f16_f32, round to nearest even), summed as f32 by v_dot2 against (1, 1)
+                    const half2_t p2 = __builtin_convertvector(
+                        (float2_t{__builtin_amdgcn_exp2f(fmaf(sc[X][2 * i], LOG2E, nm[X])),
+                                  __builtin_amdgcn_exp2f(fmaf(sc[X][2 * i + 1], LOG2E, nm[X]))}),
+                        half2_t);
+                    __builtin_memcpy(&pb[X][i], &p2, 4);
+                    l[X] = __builtin_amdgcn_fdot2(p2, half2_t{(_Float16)1.0f, (_Float16)1.0f}, l[X], false);
+                    asm volatile("" : "+v"(pb[X][i]), "+v"(l[X]));  // holds the two here
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
-            l[g] = l[g] * corr + pair_sum<32>(ps);
-            m[g] = mx;
+        };
+        static_assert(QG == 2 && AST == 2, "the turns of two groups, two blocks a stage");
+        auto turn = [&](int st) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads of stage st + 1
+            __builtin_amdgcn_s_barrier();                       // everyone's; and stage st − 1 is read by all
+            asm volatile("" ::: "memory");
+            if (st + 2 < st1) issue(st + 2);
+        };
+        auto at = [&](int st, int j) { return s_kv[st % RING] + j * (KVB / 16); };
+        // the loop body has one path, so O stays in the same registers through every iteration
+        const int to = min(st1, n_full);
+        turn(st0);
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) kread(at(st0, 0), ks);
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) score(0, ks);
+        for (int st = st0; st < to; st++) {
+            if (st > st0) turn(st);
+            step(at(st, 0), at(st, 1), 0, std::false_type{});
+            step(at(st, 1), at(st + 1, 0), 0, std::false_type{});
+        }
+        if (to < st1) {  // the last stage, with keys ≥ n_tok
+            const int st = st1 - 1, k0 = st * AST * FB;
+            if (st > st0) turn(st);
+            step(at(st, 0), at(st, 1), k0, std::true_type{});
+            if (k0 + FB < n_tok) step(at(st, 1), at(st, 1), k0 + FB, std::true_type{});
         }
 #pragma unroll
-        for (int g = 0; g < QG; g++)
+        for (int i = 0; i < 4; i++) pv(1, i);
+        __builtin_amdgcn_s_barrier();  // the next tile's first stage overwrites a buffer that another wave may still read
+        asm volatile("" ::: "memory");
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+        for (int g = 0; g < QG; g++) {
+            l[g] = pair_sum<32>(l[g]);
+            if (slot >= 0) {
+                float *p = part + (size_t)slot * PART<QG> + (size_t)(wave * QG + g) * 34 * 64 + lane;
 #pragma unroll
-                for (int st = 0; st < 2; st++)
-                    o[g][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fv[2 * t + st], pb[g][st], o[g][t], 0, 0, 0);
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) p[(16 * t + i) * 64] = o[g][t][i];
+                p[32 * 64] = nm[g];
+                p[33 * 64] = l[g];
+            } else if (q0 + FQ * g + c < n_tok) {
+                typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+                const float inv = 1.0f / l[g];
+                _Float16 *dst = O + (size_t)(q0 + FQ * g + c) * row + h * 64 + 4 * hf;
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        *reinterpret_cast<half4 *>(dst + 32 * t + 8 * r) =
+                            half4{(_Float16)(o[g][t][4 * r] * inv), (_Float16)(o[g][t][4 * r + 1] * inv),
+                                  (_Float16)(o[g][t][4 * r + 2] * inv), (_Float16)(o[g][t][4 * r + 3] * inv)};
+            }
+        }
     };
-    // stages 0 … n_full − 1 hold full blocks only: the loop body has one path, so O stays in the same registers
-    // through every iteration (a masked path inside the loop makes the compiler copy it each block)
-    const int n_stage = (n_blk + AST - 1) / AST, n_full = n_tok / (AST * FB);
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    for (int sg = 0; sg < n_full; sg++) {
-        const int buf = sg & 1;
-        if (sg + 1 < n_stage) gload(sg + 1);
-#pragma unroll
-        for (int j = 0; j < AST; j++) block(s_kv[buf] + j * (KVB / 16), (sg * AST + j) * FB, std::false_type{});
-        // the other buffer was last read in the previous stage, before the barrier that ended it
-        if (sg + 1 < n_stage) lstore(buf ^ 1);
-        __syncthreads();
+    // the worker's share of the cut tiles (it touches two at most), then its whole ones
+    const int a = sp.first(wk), b = sp.first(wk + 1), t0 = a / sp.n_stage, cut = b > a ? (b - 1) / sp.n_stage - t0 + 1 : 0;
+    const int whole = wk < sp.full ? (sp.full - 1 - wk) / sp.workers + 1 : 0;
+    for (int u = 0; u < cut + whole; u++) {
+        const int base = (t0 + u) * sp.n_stage;
+        const bool part_of = u < cut;
+        run(part_of ? sp.full + t0 + u : wk + (u - cut) * sp.workers, part_of ? max(a - base, 0) : 0,
+            part_of ? min(b - base, sp.n_stage) : sp.n_stage, part_of ? 2 * (grp * sp.workers + wk) + u : -1);
     }
-    // the last stage, when it holds keys ≥ n_tok (copied to buffer n_full % 2 by the loop's last iteration, or
-    // before the loop when n_full is 0)
-    if (n_full < n_stage) {
-        const int buf = n_full & 1;
-        for (int j = 0; j < AST; j++) {
-            const int k0 = (n_full * AST + j) * FB;
-            if (k0 + FB <= n_tok)
-                block(s_kv[buf] + j * (KVB / 16), k0, std::false_type{});
-            else if (k0 < n_tok)
-                block(s_kv[buf] + j * (KVB / 16), k0, std::true_type{});
-        }
+}
+
+// the cut tiles: the sums of the workers that share one, joined. grid (groups · cut tiles, 16·QG): a wave takes 8 of the
+// 32 registers of one (wave, query group) of the tile
+template <int QG>
+__global__ __launch_bounds__(64) void k_attn_vision_merge(const float *part, _Float16 *O, int n_tok, int n_head, VSplit sp) {
+    const int lane = threadIdx.x, hf = lane >> 5, c = lane & 31;
+    const int grp = blockIdx.x % sp.groups, t = blockIdx.x / sp.groups;
+    const int wg = blockIdx.y >> 2, r0 = 8 * (blockIdx.y & 3);  // (wave, group); the first register
+    // the workers whose shares meet stages [base, base + n_stage) of the cut tiles
+    const int base = t * sp.n_stage;
+    int w0 = (int)((long long)base * sp.workers / ((long long)(sp.tiles - sp.full) * sp.n_stage));
+    while (w0 > 0 && sp.first(w0) > base) w0--;
+    while (sp.first(w0 + 1) <= base) w0++;
+    float nm = 3.0e38f, l = 0.0f, o[8] = {};
+    for (int w = w0; w < sp.workers && sp.first(w) < base + sp.n_stage; w++) {
+        if (sp.first(w + 1) == sp.first(w)) continue;
+        const int u = t - sp.first(w) / sp.n_stage;
+        const float *p = part + (size_t)(2 * (grp * sp.workers + w) + u) * PART<QG> + (size_t)wg * 34 * 64 + lane;
+        const float pn = p[32 * 64], pl = p[33 * 64];
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = p[(r0 + e) * 64];
+        const float top = fminf(nm, pn), a = __builtin_amdgcn_exp2f(top - nm), b = __builtin_amdgcn_exp2f(top - pn);
+        nm = top;
+        l = l * a + pl * b;
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = o[e] * a + v[e] * b;
     }
+    const int tile = sp.full + t, h = grp * (n_head / sp.groups) + tile / sp.n_qt;
+    const int q = (tile % sp.n_qt) * (FWAVES * FQ * QG) + wg * FQ + c;
+    if (q >= n_tok) return;
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    const float inv = 1.0f / l;
+    // register 16t + i is dim 32t + 8(i / 4) + 4h + i % 4
+    _Float16 *dst = O + (size_t)q * n_head * 64 + h * 64 + 32 * (r0 >> 4) + 8 * ((r0 & 15) >> 2) + 4 * hf;
 #pragma unroll
-    for (int g = 0; g < QG; g++) {
-        if (q0 + FQ * g + c < n_tok) {
-            typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-            const float inv = 1.0f / l[g];
-            _Float16 *dst = O + (size_t)(q0 + FQ * g + c) * row + h * 64 + 4 * hf;
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-                    *reinterpret_cast<half4 *>(dst + 32 * t + 8 * r) =
-                        half4{(_Float16)(o[g][t][4 * r] * inv), (_Float16)(o[g][t][4 * r + 1] * inv),
-                              (_Float16)(o[g][t][4 * r + 2] * inv), (_Float16)(o[g][t][4 * r + 3] * inv)};
-        }
-    }
+    for (int r = 0; r < 2; r++)
+        *reinterpret_cast<half4 *>(dst + 8 * r) = half4{(_Float16)(o[4 * r] * inv), (_Float16)(o[4 * r + 1] * inv),
+                                                        (_Float16)(o[4 * r + 2] * inv), (_Float16)(o[4 * r + 3] * inv)};
 }
 
 // unfold2x2.wgsl: Z[o][c·4 + ky·2 + kx] = X[(2·oy + ky)·px + 2·ox + kx][c]
@@ -409,10 +483,27 @@ int launch_attn_vision(htr_device *dev, hipStream_t st, const float *q, const _F
     // two query groups a wave: 0.69 ms a layer at 12100 patches against 0.79 ms with one (223 VGPRs, 2 waves a SIMD;
     // forcing 3 spills 111 of them)
     constexpr int QG = 2;
-    const int n_qt = (n_tok + QG * FQ * FWAVES - 1) / (QG * FQ * FWAVES), n_blk = (n_tok + FB - 1) / FB;
-    hipLaunchKernelGGL(k_attn_vision<QG>, dim3(n_qt * n_head), dim3(VW), 0, st, q, kv, o, n_tok, n_head, n_blk, n_qt,
-                       scale, cs, px, max_pos);
-    return htr_launched(dev, "k_attn_vision");
+    const int n_blk = (n_tok + FB - 1) / FB;
+    VSplit sp{};
+    sp.groups = n_head % 8 == 0 ? 8 : 1;
+    sp.workers = 2 * dev->n_cu / sp.groups;
+    sp.n_qt = (n_tok + QG * FQ * FWAVES - 1) / (QG * FQ * FWAVES);
+    sp.n_stage = (n_blk + AST - 1) / AST;
+    sp.tiles = n_head / sp.groups * sp.n_qt;
+    sp.full = sp.tiles;
+    // the tiles past the full rounds are cut where that shortens the last round by more than the merge costs
+    const int left = sp.tiles % sp.workers;
+    if (left && (left * sp.n_stage + sp.workers - 1) / sp.workers + CUT_COST < sp.n_stage) sp.full -= left;
+    float *part = nullptr;
+    if (sp.full < sp.tiles)
+        HTR_TRY(htr_scratch(dev, SCR_VISION_PART, (size_t)2 * sp.groups * sp.workers * PART<QG> * 4, (void **)&part));
+    hipLaunchKernelGGL(k_attn_vision<QG>, dim3(sp.groups * sp.workers), dim3(VW), 0, st, q, kv, o, n_tok, n_head, n_blk, sp,
+                       scale, cs, px, max_pos, part);
+    HTR_TRY(htr_launched(dev, "k_attn_vision"));
+    if (sp.full == sp.tiles) return 0;
+    hipLaunchKernelGGL(k_attn_vision_merge<QG>, dim3(sp.groups * (sp.tiles - sp.full), 16 * QG), dim3(64), 0, st, part, o,
+                       n_tok, n_head, sp);
+    return htr_launched(dev, "k_attn_vision_merge");
 }
 
 int launch_unfold2x2(htr_device *dev, hipStream_t st, const float *x, float *z, int px, int py, int dim) {

@@ -40,6 +40,17 @@ def test_tiny_encoder_matches_oracle(tiny, w, h):
         assert e < (1e-5 if nl == 0 else 2e-4), nl
 
 
+# attention tiles cut along their keys and joined: key stages 14, 21 and 24 (64 keys each) shared by one to a few workers,
+# the last stage ragged or whole, queries that do not fill the last tile
+@pytest.mark.parametrize("w,h", [(308, 560), (420, 616), (196, 1512)])
+def test_tiny_encoder_on_cut_attention_tiles_matches_oracle(tiny, w, h):
+    cfg, t, v = tiny
+    rgb = tiny_page(cfg, w, h, seed=w + h)
+    e = rel_l2(v.encode(rgb, 1), orc.vision_encode(cfg, t, rgb, 1))
+    print(f"\n[vision {w}x{h} layers 1] rel-L2 vs oracle {e:.2e}")
+    assert e < 2e-4  # the bar of the tiny encoders' first layer
+
+
 def test_encoder_rejects_unbaked_pages(tiny):
     cfg, t, v = tiny
     with pytest.raises(htr.HtrError, match="not baked"):
