@@ -324,6 +324,127 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const in
     }
 }
 
+// ---- few rows ----------------------------------------------------------------------------------------------------------
+//
+// The same products for at most 32 rows. The tiles above make a call of that size a chain of conversions and stage
+// latencies on a handful of CUs (a 64 × 64 tile converts mostly rows that are not there); here a workgroup owns 32 columns
+// and its 8 waves split K: each takes a contiguous run of q8_0 blocks straight from memory into MFMA fragments (no LDS, no
+// barrier; 3 blocks of loads in flight), and the waves' sums are added in order through LDS. Inside a block lane half h
+// takes k 16h … 16h + 15 for both MFMA steps (any order of k serves that X and W share), so a lane's quants are one 16-byte
+// load and its X values one 64-byte run: 32 rows are 64 lines a load, which is what bounds it and why it stops at 32.
+constexpr int FEW_WAVES = 8, FEW_R = 3;
+
+template <bool EX>
+__global__ __launch_bounds__(64 * FEW_WAVES) void k_gemm_q8_0_few(const float *x, const int8_t *wq, const _Float16 *wd,
+                                                                  float *y, int m, int n, int k, int acc, int al) {
+    __shared__ float s_o[FEW_WAVES][32][32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col0 = blockIdx.x * 32, r32 = lane & 31, hk = lane >> 5, nb = k / 32;
+    const int per = (nb + FEW_WAVES - 1) / FEW_WAVES, b0 = min(per * wave, nb), b1 = min(b0 + per, nb);
+    const size_t wr = min(col0 + r32, n - 1);
+    const int8_t *q = wq + wr * k + 16 * hk;
+    const _Float16 *d = wd + wr * nb;
+    const float *xr = x + (size_t)min(r32, m - 1) * k + 16 * hk;
+    struct Regs {
+        float4 a[4];
+        int4 q;
+        _Float16 d;
+    } ring[FEW_R];
+    auto gload = [&](Regs &r, int b) {
+        b = max(min(b, b1 - 1), 0);
+        const float *xs = xr + 32 * b;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            r.a[i] = al ? reinterpret_cast<const float4 *>(xs)[i]
+                        : make_float4(xs[4 * i], xs[4 * i + 1], xs[4 * i + 2], xs[4 * i + 3]);
+        r.q = *reinterpret_cast<const int4 *>(q + 32 * b);
+        r.d = d[b];
+    };
+    f32x16 c = {};
+    auto use = [&](const Regs &r) {
+        const int2 qs[2] = {make_int2(r.q.x, r.q.y), make_int2(r.q.z, r.q.w)};
+        if constexpr (EX) {
+            bf16x8 b[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                uint32_t f[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) f[e] = __float_as_uint((float)q_byte(qs[h], e));
+                const int4 v = make_int4((int)hi_pair(f[0], f[1]), (int)hi_pair(f[2], f[3]), (int)hi_pair(f[4], f[5]),
+                                         (int)hi_pair(f[6], f[7]));
+                __builtin_memcpy(&b[h], &v, 16);
+            }
+            f32x16 p;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const float4 u = r.a[2 * h], v = r.a[2 * h + 1];
+                const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+                int4 a[3];
+                split3(f, a);
+#pragma unroll
+                for (int pl = 0; pl < 3; pl++) {
+                    bf16x8 av;
+                    __builtin_memcpy(&av, &a[pl], 16);
+                    p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, b[h], h + pl ? p : f32x16{}, 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) c[i] = fmaf(p[i], (float)r.d, c[i]);
+        } else {
+            const float ds = (float)r.d;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                half2_t w[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    w[e] = __builtin_convertvector(
+                        (float2_t{(float)q_byte(qs[h], 2 * e) * ds, (float)q_byte(qs[h], 2 * e + 1) * ds}), half2_t);
+                half8 b;
+                __builtin_memcpy(&b, w, 16);
+                const float4 u = r.a[2 * h], v = r.a[2 * h + 1];
+                const half2_t a4[4] = {__builtin_convertvector((float2_t{u.x, u.y}), half2_t),
+                                       __builtin_convertvector((float2_t{u.z, u.w}), half2_t),
+                                       __builtin_convertvector((float2_t{v.x, v.y}), half2_t),
+                                       __builtin_convertvector((float2_t{v.z, v.w}), half2_t)};
+                half8 a;
+                __builtin_memcpy(&a, a4, 16);
+                c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+            }
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < FEW_R; i++) gload(ring[i], b0 + i);
+    for (int i0 = b0; i0 < b1; i0 += FEW_R) {
+#pragma unroll
+        for (int i = 0; i < FEW_R; i++)
+            if (i0 + i < b1) {
+                use(ring[i]);
+                gload(ring[i], i0 + i + FEW_R);
+            }
+    }
+    // lane ℓ, register r: row 8(r/4) + 4(ℓ/32) + r%4, column ℓ%32
+#pragma unroll
+    for (int i = 0; i < 16; i++) s_o[wave][8 * (i >> 2) + 4 * hk + (i & 3)][r32] = c[i];
+    __syncthreads();
+    constexpr int NE = 32 * 32 / (64 * FEW_WAVES);
+    float old[NE];
+    if (acc) {  // every load before the first store, which may alias them
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            const int o = tid + 64 * FEW_WAVES * e;
+            old[e] = y[(size_t)min(o / 32, m - 1) * n + min(col0 + o % 32, n - 1)];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+        const int o = tid + 64 * FEW_WAVES * e, row = o / 32, col = col0 + o % 32;
+        float v = s_o[0][o / 32][o % 32];
+#pragma unroll
+        for (int g = 1; g < FEW_WAVES; g++) v += s_o[g][o / 32][o % 32];
+        if (row < m && col < n) y[(size_t)row * n + col] = acc ? old[e] + v : v;
+    }
+}
+
 // ---- the F32 path's K and V projections --------------------------------------------------------------------------------
 //
 // Y = X·Wᵀ with every output one chain of f32 fmas over k in order (matmul.wgsl:47-91), bit for bit: v_mfma_f32_16x16x4_f32
@@ -484,8 +605,18 @@ template <bool EX> int gemm_q8(htr_device *dev, hipStream_t st, const float *x, 
     if (!w->q) return htr_fail("gemm: weight has no q8_0 planes");
     const int n = (int)w->rows;
     const long t128 = (long)((m + 127) / 128) * ((n + 127) / 128), t64 = (long)((m + 63) / 64) * ((n + 63) / 64);
+    // few rows on one round of workgroups (µs a call, tiles → few; f16: 1 × 1024 × 1024 8.6 → 6.2, 8 × 1024 × 3072 17.4 →
+    // 14.0, 12 × 1024 × 1024 8.7 → 8.0, 16 rows even, 24 8.7 → 9.8; F32: 1 × 1024 × 1024 11.3 → 6.4, 8 × 1024 × 3072 27.4 →
+    // 14.6, 32 × 1024 × 2048 19.7 → 16.2; 16 × 16384 × 1024, two rounds: 9.7 → 16.2 and 13.1 → 16.4)
+    if (m <= (EX ? 32 : 12) && (n + 31) / 32 <= dev->n_cu) {
+        hipLaunchKernelGGL(k_gemm_q8_0_few<EX>, dim3((n + 31) / 32), dim3(64 * FEW_WAVES), 0, st, x, w->q, w->d, y, m, n,
+                           (int)w->cols, acc, (int)((uintptr_t)x % 16 == 0));
+        return htr_launched(dev, EX ? "k_gemm_q8_0_few<f32>" : "k_gemm_q8_0_few<f16>");
+    }
+    // 128 × 128 tiles from one a CU on; of the 64 × 64 ones, 4 K groups while every CU has a tile at most, else 2, whose
+    // workgroups go two to a CU (288 tiles, 333 × 3072 × 1024: f16 18.5 → 14.2 µs, F32 24.1 → 21.8)
     if (t128 >= dev->n_cu) launch_q8<EX, 2, 1>(dev, st, x, w, y, m, acc);
-    else if (t64 >= 2 * dev->n_cu) launch_q8<EX, 1, 2>(dev, st, x, w, y, m, acc);
+    else if (t64 > dev->n_cu) launch_q8<EX, 1, 2>(dev, st, x, w, y, m, acc);
     else launch_q8<EX, 1, 4>(dev, st, x, w, y, m, acc);
     return htr_launched(dev, EX ? "k_gemm_q8_0<f32>" : "k_gemm_q8_0<f16>");
 }

@@ -269,6 +269,14 @@ def test_matmul_q8_0_tiles_against_fp64(dev, m, n, k, off):
     w.free()
 
 
+# either side of the few-row kernel's rules (12 and 32 rows, one round of 32-column workgroups), waves with no block of K
+# and with an uneven share, a last column tile cut, X off the 16-byte grid
+@pytest.mark.parametrize("m,n,k,off", [(12, 65, 96, 4), (13, 33, 288, 0), (32, 1000, 3072, 0), (33, 64, 64, 0), (5, 8193, 64, 0),
+                                       (32, 31, 352, 8), (333, 3072, 64, 0)])
+def test_matmul_q8_0_few_rows_against_fp64(dev, m, n, k, off):
+    test_matmul_q8_0_tiles_against_fp64(dev, m, n, k, off)
+
+
 def test_matmul_q8_0_f32_path_keeps_infinities_and_nans(dev):
     """one infinity a row gives ±inf (NaN where its quant is 0), a NaN a NaN — also one whose payload is in its low
     half — and the largest finite values stay exact; the other rows are untouched"""
