@@ -155,14 +155,15 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const in
 #pragma unroll
         for (int i = 0; i < UN; i++) {
             const int u = tid + 256 * i, rr = u / CPR, c = u % CPR, at = q8_slot<CPR>(rr, c);
-            const bool in = st * KB + c / 4 < nb;
             const float4 a0 = r.a[i][0], a1 = r.a[i][1];
             float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-            if (!in) {
+            float d = (float)r.d[i];
+            if ((st + 1) * KB > nb) {  // only a stage that runs past the last block pays for the zeros
+                const bool in = st * KB + c / 4 < nb;
 #pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = 0.0f;
+                for (int e = 0; e < 8; e++) v[e] = in ? v[e] : 0.0f;
+                d = in ? d : 0.0f;
             }
-            const float d = in ? (float)r.d[i] : 0.0f;
             if constexpr (EX) {
                 int4 p[3];
                 split3(v, p);
