@@ -10,12 +10,12 @@
 //             TM × TN v_mfma_f32_32x32x16_f16 tiles (lane layouts checked on the GPU: A lane ℓ holds
 //             A[ℓ%32][8(ℓ/32) …+7], B lane ℓ holds B[8(ℓ/32) …+7][ℓ%32], D lane ℓ register r is row 8(r/4) + 4(ℓ/32)
 //             + r%4, column ℓ%32). Tile shapes: 256 × 256 and 192 × 256 (8 waves of 128 × 64 / 96 × 64), 128 × 128
-//             and 64 × 64 (4 waves of 64 × 64 / 32 × 32); the launch takes the largest that still gives half a
+//             (8 waves of 32 × 64; the FFN 4 of 64 × 64) and 64 × 64 (4 waves of 32 × 32); the launch takes the largest that still gives half a
 //             workgroup per CU, 192 rows where that takes fewer rows × rounds, and splits K for prompt-sized M.
 //             The FFN's W tile is BN/2 gate rows and the same BN/2 up rows in alternating blocks of 32, so a wave's
 //             two column tiles are one gate and one up tile of the same outputs;
 //   K         through a ring of LDS stages filled by direct-to-LDS loads (global_load_lds_dwordx4): the 256-wide
-//             tiles in stages of 64 (a row's 128 bytes of the stage, whole cache lines) in a ring of 2, the stage
+//             tiles and the FFN's 128-wide one in stages of 64 (a row's 128 bytes of the stage, whole cache lines) in a ring of 2, the stage
 //             after next loading while one is computed; the smaller tiles in stages of 32 in a ring of 4, the stage
 //             3 ahead loading. Inside a stage a row's 16-byte chunks sit XOR-placed (chunk ^ (row/4 % 4) for 4 a
 //             row, chunk ^ (row/2 % 8) for 8): 16 consecutive rows of one chunk fall on 16 different 16-byte bank
@@ -60,7 +60,8 @@ template <int BM_, int BN_, int WM_, int WN_, int AM_ = BM_, int KS_ = 32, int N
 };
 using T256 = Tile<256, 256, 2, 4, 256, 64, 2>;
 using T192 = Tile<192, 256, 2, 4, 256, 64, 2>;
-using T128 = Tile<128, 128, 2, 2>;
+using T128 = Tile<128, 128, 4, 2>;   // 8 waves: with a workgroup a CU two a SIMD (1023 × 4096 × 1024 18.4 → 17.7 µs)
+using T128F = Tile<128, 128, 2, 2, 128, 64, 2>;
 using T64 = Tile<64, 64, 2, 2>;
 
 constexpr int GROUP = 4;   // tile rows walked together
@@ -513,10 +514,11 @@ int launch(htr_device *dev, hipStream_t st, int epi, GemmK &a, bool *normed = nu
         }
     }
     // too few 256 / 128 tiles and a long K (one weight; N a multiple of 4): 128 × 128 tiles with K split over up to 4
-    // workgroups (a multiple of 32 each), the products summed in split order by k_split_reduce
+    // workgroups (a multiple of 32 each), the products summed in split order by k_split_reduce. A very long K also where
+    // two workgroups a tile are about one a CU (2145 × 1024 × 8192, the projector's merger: 87 → 67 + 6 µs)
     a.split = 1;
-    if (pick != 0 && epi != GEMM_FFN && a.n_w == 1 && a.rows[0] % 4 == 0 && n_tiles[1] > 0 && n_tiles[1] < want &&
-        a.k >= 1024) {
+    if (pick != 0 && epi != GEMM_FFN && a.n_w == 1 && a.rows[0] % 4 == 0 && n_tiles[1] > 0 &&
+        ((n_tiles[1] < want && a.k >= 1024) || (16 * n_tiles[1] <= 9 * dev->n_cu && a.k >= 4096))) {
         int sp = std::min(4, (dev->n_cu + n_tiles[1] - 1) / n_tiles[1]);
         while (sp > 1 && a.k % (32 * sp)) sp--;
         if (sp > 1) {
@@ -560,7 +562,12 @@ int launch(htr_device *dev, hipStream_t st, int epi, GemmK &a, bool *normed = nu
     }
     if (pick == 1) {
         tiles_for<T128>(a, epi, a.tiles_m, a.tiles_n);
-        launch_tile<T128>(st, epi, a);
+        // the FFN's waves pair a gate and an up tile, so 8 waves would hold 32 × 64 each and read three fragments for two
+        // MFMAs: 4 waves with stages of 64 instead (1023 × 6144 × 1024 24.7 → 21.5 µs, 8 waves 24.4)
+        if (epi == GEMM_FFN && a.k % 64 == 0)
+            hipLaunchKernelGGL((k_gemm_f16<GEMM_FFN, T128F, false>), dim3(a.tiles_m * a.tiles_n), dim3(T128F::GW), 0, st, a);
+        else
+            launch_tile<T128>(st, epi, a);
         return htr_launched(dev, "k_gemm_f16<128>");
     }
     tiles_for<T64>(a, epi, a.tiles_m, a.tiles_n);
