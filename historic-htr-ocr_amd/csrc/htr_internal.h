@@ -257,8 +257,11 @@ const char *ggml_type_name(uint32_t ty);
 std::string gguf_shape_str(const GgufTensor &t);  // "[a, b, …]"
 
 // the vision encoder's other kernels (vision.hip)
-int launch_patchify(htr_device *dev, hipStream_t st, const uint8_t *rgb, const float *lut, int w, int px, int n,
-                    int side, float *P);
+// the image's patches as [hi | hi | lo] rows of segments of kp; the projector's normed, unfolded input as [hi | lo] rows
+int launch_patchify_split(htr_device *dev, hipStream_t st, const uint8_t *rgb, const float *lut, int w, int px, int n,
+                          int side, int kp, _Float16 *out);
+int launch_norm_unfold_split(htr_device *dev, hipStream_t st, const float *x, const float *w, int px, int py, int dim,
+                             float eps, _Float16 *out);
 int launch_rms_norm_f16(htr_device *dev, hipStream_t st, const float *x, const float *w, _Float16 *y, int rows, int dim,
                         float eps);
 // K / V of the vision attention as f16 key blocks of 8 KB per head (vision_kv_bytes in all)
@@ -267,11 +270,10 @@ int launch_heads_f16(htr_device *dev, hipStream_t st, const float *k, const floa
 size_t vision_kv_bytes(int n_tok, int n_head);
 int launch_attn_vision(htr_device *dev, hipStream_t st, const float *q, const _Float16 *kv, _Float16 *o, int n_tok,
                        int n_head, float scale, const float *cs, int px, int max_pos);
-int launch_unfold2x2(htr_device *dev, hipStream_t st, const float *x, float *z, int px, int py, int dim);
-int launch_gelu(htr_device *dev, hipStream_t st, float *x, size_t n);
-// x f32 [m][k] → f16 rows of nseg segments of kp values: hi = f16(x), or lo = f16(x − hi) in the segments of lo_mask
+// x (or gelu(x)) f32 [m][k] → f16 rows of nseg segments of kp values: hi = f16(x), or lo = f16(x − hi) in the segments of
+// lo_mask
 int launch_split_f16(htr_device *dev, hipStream_t st, const float *x, int m, int k, int kp, int nseg, int lo_mask,
-                     _Float16 *out);
+                     _Float16 *out, bool of_gelu = false);
 
 // the decode step of the 1024 / 2048 / 3072 decoder as one launch per token (token_step.hip)
 struct TokLayer {

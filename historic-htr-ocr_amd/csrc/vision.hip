@@ -19,16 +19,29 @@ constexpr int VW = 256;
 __device__ __forceinline__ size_t gsize() { return (size_t)gridDim.x * VW; }
 __device__ __forceinline__ size_t gid() { return blockIdx.x * (size_t)VW + threadIdx.x; }
 
-// patchify.wgsl: P[t][c·p·p + ky·p + kx] = lut[c·256 + rgb[((ty·p + ky)·w + tx·p + kx)·3 + c]]
-__global__ __launch_bounds__(VW) void k_patchify(const uint8_t *rgb, const float *lut, int w, int px, int n, int side,
-                                                 float *P) {
-    const int pp = side * side;
-    const size_t total = (size_t)n * 3 * pp;
-    for (size_t i = gid(); i < total; i += gsize()) {
-        const int t = (int)(i / (3 * pp)), r = (int)(i % (3 * pp));
-        const int c = r / pp, ky = (r % pp) / side, kx = r % side;
-        const int x = (t % px) * side + kx, y = (t / px) * side + ky;
-        P[i] = lut[c * 256 + rgb[((size_t)y * w + x) * 3 + c]];
+// x as f16 pieces: hi = f16(x), lo = f16(x − hi)
+__device__ __forceinline__ void split_hi_lo(float v, _Float16 &hi, _Float16 &lo) {
+    hi = (_Float16)v;
+    lo = (_Float16)(v - (float)hi);
+}
+
+// patchify.wgsl, P[t][c·p·p + ky·p + kx] = lut[c·256 + rgb[((ty·p + ky)·w + tx·p + kx)·3 + c]], straight into the pieces
+// [hi | hi | lo] that the patch embedding multiplies (k_split_f16's layout, segments of kp): a patch a workgroup. The
+// bytes of a patch and its 3·kp halves are all that moves; patches written as f32 and split by a second kernel took
+// 24 + 20 µs for 8580 of them, this 21 µs
+__global__ __launch_bounds__(VW) void k_patchify_split(const uint8_t *rgb, const float *lut, int w, int px, int side, int kp,
+                                                       _Float16 *out) {
+    const int t = blockIdx.x, pp = side * side;
+    const uint8_t *src = rgb + ((size_t)(t / px) * side * w + (size_t)(t % px) * side) * 3;
+    _Float16 *dst = out + (size_t)t * 3 * kp;
+    for (int r = threadIdx.x; r < kp; r += VW) {
+        const int c = r / pp, i = r % pp;
+        const float v = r < 3 * pp ? lut[c * 256 + src[((size_t)(i / side) * w + i % side) * 3 + c]] : 0.0f;
+        _Float16 hi, lo;
+        split_hi_lo(v, hi, lo);
+        dst[r] = hi;
+        dst[kp + r] = hi;
+        dst[2 * kp + r] = lo;
     }
 }
 
@@ -404,39 +417,72 @@ __global__ __launch_bounds__(64) void k_attn_vision_merge(const float *part, _Fl
                                                         (_Float16)(o[4 * r + 2] * inv), (_Float16)(o[4 * r + 3] * inv)};
 }
 
-// unfold2x2.wgsl: Z[o][c·4 + ky·2 + kx] = X[(2·oy + ky)·px + 2·ox + kx][c]
-__global__ __launch_bounds__(VW) void k_unfold2x2(const float *X, float *Z, int px, int py, int dim) {
-    const int ox_n = px / 2;
-    const size_t total = (size_t)(px / 2) * (py / 2) * dim * 4;
-    for (size_t i = gid(); i < total; i += gsize()) {
-        const int kx = (int)(i % 2), ky = (int)((i / 2) % 2), c = (int)((i / 4) % dim);
-        const int o = (int)(i / (4 * (size_t)dim));
-        const int ox = o % ox_n, oy = o / ox_n;
-        Z[i] = X[((size_t)(2 * oy + ky) * px + 2 * ox + kx) * dim + c];
+// the projector's input: rows normed (y = x·1/sqrt(mean(x²) + eps)·w), unfold2x2.wgsl, Z[o][c·4 + ky·2 + kx] =
+// Y[(2·oy + ky)·px + 2·ox + kx][c], as the pieces [hi | lo] (k_split_f16's layout): an output row a workgroup, which reads
+// its four patches twice (the second time from the caches) and writes 8 bytes a channel and piece. Norm, unfold and split
+// as three kernels took 18 + 29 + 26 µs for 8580 rows of 1024, this 19 µs
+__global__ __launch_bounds__(VW) void k_norm_unfold_split(const float *X, const float *w, int px, int dim, float eps,
+                                                          _Float16 *out) {
+    __shared__ float red[4][VW / 64];
+    const int o = blockIdx.x, tid = threadIdx.x, lane = tid & 63, ox = o % (px / 2), oy = o / (px / 2);
+    const float *x[4];
+    float s[4] = {}, scale[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) x[j] = X + ((size_t)(2 * oy + (j >> 1)) * px + 2 * ox + (j & 1)) * dim;
+    for (int c = tid; c < dim; c += VW)
+#pragma unroll
+        for (int j = 0; j < 4; j++) s[j] = fmaf(x[j][c], x[j][c], s[j]);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        s[j] = wave_sum(s[j], lane);
+        if (lane == 0) red[j][tid >> 6] = s[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        scale[j] = 1.0f / sqrtf(((red[j][0] + red[j][1]) + (red[j][2] + red[j][3])) / (float)dim + eps);
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    half4 *hi = reinterpret_cast<half4 *>(out + (size_t)o * 8 * dim), *lo = hi + dim;
+    for (int c = tid; c < dim; c += VW) {
+        half4 h, l;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float v = (x[j][c] * scale[j]) * w[c];
+            asm volatile("" : "+v"(v));  // one f32 value for both pieces
+            _Float16 a, b;
+            split_hi_lo(v, a, b);
+            h[j] = a, l[j] = b;
+        }
+        hi[c] = h;
+        lo[c] = l;
     }
 }
 
-// gelu.wgsl in place (tanh form, argument clamped to ±15)
-__global__ __launch_bounds__(VW) void k_gelu(float *X, size_t n) {
-    for (size_t i = gid(); i < n; i += gsize()) {
-        const float x = X[i];
-        const float t = fminf(fmaxf(0.7978845608028654f * x * (1.0f + 0.044715f * x * x), -15.0f), 15.0f);
-        X[i] = 0.5f * x * (1.0f + tanhf(t));
-    }
+// gelu.wgsl (tanh form, argument clamped to ±15)
+__device__ __forceinline__ float gelu(float x) {
+    const float t = fminf(fmaxf(0.7978845608028654f * x * (1.0f + 0.044715f * x * x), -15.0f), 15.0f);
+    return 0.5f * x * (1.0f + tanhf(t));
 }
 
 // f32 values as f16 pieces for f32-grade products on the f16 matrix cores: x [m][k] → rows of nseg segments of kp
 // values (kp ≥ k, a multiple of 32, the values past k zero); segment s holds hi = f16(x), or lo = f16(x − hi) where bit
 // s of lo_mask is set. x − hi is exact in f32 and hi + lo is x within 2^-22·|x| (|x| < 65504). With X as [hi, hi, lo]
 // and W as [hi, lo, hi] one f16 GEMM over 3·kp sums xh·wh + xh·wl + xl·wh in f32; f16-valued W: X [hi, lo], W [w, w].
+// GELU: of gelu(x)
+template <bool GELU>
 __global__ __launch_bounds__(VW) void k_split_f16(const float *x, int m, int k, int kp, int nseg, int lo_mask,
                                                   _Float16 *out) {
     const size_t total = (size_t)m * kp;
     for (size_t i = gid(); i < total; i += gsize()) {
         const int c = (int)(i % kp);
         const size_t r = i / kp;
-        const float v = c < k ? x[r * k + c] : 0.0f;
-        const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
+        float v = c < k ? x[r * k + c] : 0.0f;
+        if (GELU) {
+            v = gelu(v);
+            asm volatile("" : "+v"(v));  // one f32 value for both pieces
+        }
+        _Float16 hi, lo;
+        split_hi_lo(v, hi, lo);
         for (int s = 0; s < nseg; s++) out[(r * nseg + s) * kp + c] = (lo_mask >> s) & 1 ? lo : hi;
     }
 }
@@ -445,11 +491,11 @@ int grid_for(size_t total) { return (int)std::max<size_t>(1, std::min<size_t>((t
 
 }  // namespace
 
-int launch_patchify(htr_device *dev, hipStream_t st, const uint8_t *rgb, const float *lut, int w, int px, int n,
-                    int side, float *P) {
-    hipLaunchKernelGGL(k_patchify, dim3(grid_for((size_t)n * 3 * side * side)), dim3(VW), 0, st, rgb, lut, w, px, n,
-                       side, P);
-    return htr_launched(dev, "k_patchify");
+int launch_patchify_split(htr_device *dev, hipStream_t st, const uint8_t *rgb, const float *lut, int w, int px, int n,
+                          int side, int kp, _Float16 *out) {
+    if (n < 1 || kp < 3 * side * side) return htr_fail("patchify: %d patches of side %d in segments of %d", n, side, kp);
+    hipLaunchKernelGGL(k_patchify_split, dim3(n), dim3(VW), 0, st, rgb, lut, w, px, side, kp, out);
+    return htr_launched(dev, "k_patchify_split");
 }
 
 int launch_rms_norm_f16(htr_device *dev, hipStream_t st, const float *x, const float *w, _Float16 *y, int rows, int dim,
@@ -506,20 +552,18 @@ int launch_attn_vision(htr_device *dev, hipStream_t st, const float *q, const _F
     return htr_launched(dev, "k_attn_vision_merge");
 }
 
-int launch_unfold2x2(htr_device *dev, hipStream_t st, const float *x, float *z, int px, int py, int dim) {
-    hipLaunchKernelGGL(k_unfold2x2, dim3(grid_for((size_t)px * py * dim)), dim3(VW), 0, st, x, z, px, py, dim);
-    return htr_launched(dev, "k_unfold2x2");
-}
-
-int launch_gelu(htr_device *dev, hipStream_t st, float *x, size_t n) {
-    hipLaunchKernelGGL(k_gelu, dim3(grid_for(n)), dim3(VW), 0, st, x, n);
-    return htr_launched(dev, "k_gelu");
+int launch_norm_unfold_split(htr_device *dev, hipStream_t st, const float *x, const float *w, int px, int py, int dim,
+                             float eps, _Float16 *out) {
+    hipLaunchKernelGGL(k_norm_unfold_split, dim3((px / 2) * (py / 2)), dim3(VW), 0, st, x, w, px, dim, eps, out);
+    return htr_launched(dev, "k_norm_unfold_split");
 }
 
 int launch_split_f16(htr_device *dev, hipStream_t st, const float *x, int m, int k, int kp, int nseg, int lo_mask,
-                     _Float16 *out) {
+                     _Float16 *out, bool of_gelu) {
     if (m < 1 || k < 1 || kp < k || kp % 32 || nseg < 1 || nseg > 3)
         return htr_fail("split_f16: [%d x %d] into %d segments of %d", m, k, nseg, kp);
-    hipLaunchKernelGGL(k_split_f16, dim3(grid_for((size_t)m * kp)), dim3(VW), 0, st, x, m, k, kp, nseg, lo_mask, out);
+    const dim3 grid(grid_for((size_t)m * kp));
+    if (of_gelu) hipLaunchKernelGGL(k_split_f16<true>, grid, dim3(VW), 0, st, x, m, k, kp, nseg, lo_mask, out);
+    else hipLaunchKernelGGL(k_split_f16<false>, grid, dim3(VW), 0, st, x, m, k, kp, nseg, lo_mask, out);
     return htr_launched(dev, "k_split_f16");
 }

@@ -49,7 +49,7 @@ struct htr_vision {
     int n_cap = 0, pos_cap = 0;
     uint8_t *rgb = nullptr;
     size_t rgb_cap = 0;
-    float *P = nullptr, *x = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *tmp = nullptr, *cs = nullptr;
+    float *x = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *tmp = nullptr, *cs = nullptr;
     _Float16 *h16 = nullptr, *a16 = nullptr, *g16 = nullptr, *kv = nullptr;
     // the f32 operands of the patch embedding and the projector as f16 pieces (k_split_f16): the patch embedding
     // weight [dim][hi | lo | hi] in segments of pe_kp (the patch's 3·p² values padded to a multiple of 32); the
@@ -112,26 +112,25 @@ int split_patch_embd(htr_vision *v, size_t pp) {
 }
 
 void free_bufs(htr_vision *v) {
-    for (void *p : {(void *)v->rgb, (void *)v->P, (void *)v->x, (void *)v->q, (void *)v->k, (void *)v->v, (void *)v->tmp,
+    for (void *p : {(void *)v->rgb, (void *)v->x, (void *)v->q, (void *)v->k, (void *)v->v, (void *)v->tmp,
                     (void *)v->cs, (void *)v->h16, (void *)v->a16, (void *)v->g16, (void *)v->kv, (void *)v->xs})
         if (p) htr_dev_free(v->dev, p);
     v->rgb = nullptr;
-    v->P = v->x = v->q = v->k = v->v = v->tmp = v->cs = nullptr;
+    v->x = v->q = v->k = v->v = v->tmp = v->cs = nullptr;
     v->h16 = v->a16 = v->g16 = v->kv = v->xs = nullptr;
     v->n_cap = v->pos_cap = 0;
     v->rgb_cap = 0;
 }
 
-// buffers for n patches (and the projector: unfold n·dim, merged n/4·dim, mm.1 n/4·proj_dim fit in q / k / v)
+// buffers for n patches (and the projector: merged n/4·dim, mm.1 n/4·proj_dim fit in k / v)
 int ensure_bufs(htr_vision *v, int n, int max_pos, size_t rgb_bytes) {
     const htr_vision_config &c = v->cfg;
     htr_device *dev = v->dev;
     if (n > v->n_cap || max_pos > v->pos_cap || rgb_bytes > v->rgb_cap) {
         free_bufs(v);
-        const size_t d = c.dim, f = c.n_ff, pp = 3 * (size_t)c.patch * c.patch;
+        const size_t d = c.dim, f = c.n_ff;
         const size_t qkv = (size_t)n * std::max<size_t>(d, (size_t)c.proj_dim);
         int rc = htr_dev_alloc(dev, rgb_bytes, HTR_MEM_WORK, (void **)&v->rgb);
-        if (rc == 0) rc = htr_dev_alloc(dev, (size_t)n * pp * 4, HTR_MEM_WORK, (void **)&v->P);
         if (rc == 0) rc = htr_dev_alloc(dev, (size_t)n * d * 4, HTR_MEM_WORK, (void **)&v->x);
         if (rc == 0) rc = htr_dev_alloc(dev, qkv * 4, HTR_MEM_WORK, (void **)&v->q);
         if (rc == 0) rc = htr_dev_alloc(dev, qkv * 4, HTR_MEM_WORK, (void **)&v->k);
@@ -435,7 +434,7 @@ extern "C" int htr_vision_encode(htr_vision *v, const uint8_t *h_rgb, int width,
     HTR_TRY(htr_check_alive(dev));
     HTR_TRY(htr_vision_out_shape(v, width, height, n_layers, nullptr, nullptr));
     const htr_vision_config &c = v->cfg;
-    const int px = width / c.patch, py = height / c.patch, n = px * py, d = c.dim, pp = 3 * c.patch * c.patch;
+    const int px = width / c.patch, py = height / c.patch, n = px * py, d = c.dim;
     const int max_pos = std::max(px, py);
     const size_t rgb_bytes = (size_t)width * height * 3;
     HTR_TRY(ensure_bufs(v, n, max_pos, rgb_bytes));
@@ -445,9 +444,8 @@ extern "C" int htr_vision_encode(htr_vision *v, const uint8_t *h_rgb, int width,
     HTR_TRY(htr_upload(dev, v->cs, cs.data(), cs.size() * 4));
     const float scale = 1.0f / sqrtf((float)c.d_head);
     const int nl = n_layers < 0 ? c.n_layer : n_layers;
-    HTR_TRY(launch_patchify(dev, st, v->rgb, v->lut, width, px, n, c.patch, v->P));
     // the patch embedding in f32 grade: [xh | xh | xl]·[wh | wl | wh]ᵀ
-    HTR_TRY(launch_split_f16(dev, st, v->P, n, pp, v->pe_kp, 3, 0b100, v->xs));
+    HTR_TRY(launch_patchify_split(dev, st, v->rgb, v->lut, width, px, n, c.patch, v->pe_kp, v->xs));
     HTR_TRY(launch_gemm_f16(dev, st, GEMM_F32, v->xs, n, v->pe, nullptr, v->tmp, nullptr, 1.0f));
     HTR_TRY(launch_rms_norm(dev, st, v->tmp, v->pre_ln, v->x, n, d, c.eps));
     for (int li = 0; li < nl; li++) {
@@ -474,15 +472,12 @@ extern "C" int htr_vision_encode(htr_vision *v, const uint8_t *h_rgb, int width,
     }
     // project (vision.rs:405-423): input_norm → unfold 2×2 → merger → mm.1 → gelu → mm.2
     const int n_out = n / 4;
-    HTR_TRY(launch_rms_norm(dev, st, v->x, v->input_norm, v->tmp, n, d, c.eps));
-    HTR_TRY(launch_unfold2x2(dev, st, v->tmp, v->q, px, py, d));
     // the projector's f32 activations as [hi | lo] against its weights [w | w]
-    HTR_TRY(launch_split_f16(dev, st, v->q, n_out, 4 * d, 4 * d, 2, 0b10, v->xs));
+    HTR_TRY(launch_norm_unfold_split(dev, st, v->x, v->input_norm, px, py, d, c.eps, v->xs));
     HTR_TRY(launch_gemm_f16(dev, st, GEMM_F32, v->xs, n_out, v->merger, nullptr, v->k, nullptr, 1.0f));
     HTR_TRY(launch_split_f16(dev, st, v->k, n_out, d, d, 2, 0b10, v->xs));
     HTR_TRY(launch_gemm_f16(dev, st, GEMM_F32, v->xs, n_out, v->mm1, nullptr, v->v, nullptr, 1.0f));
-    HTR_TRY(launch_gelu(dev, st, v->v, (size_t)n_out * c.proj_dim));
-    HTR_TRY(launch_split_f16(dev, st, v->v, n_out, c.proj_dim, c.proj_dim, 2, 0b10, v->xs));
+    HTR_TRY(launch_split_f16(dev, st, v->v, n_out, c.proj_dim, c.proj_dim, 2, 0b10, v->xs, true));
     HTR_TRY(launch_gemm_f16(dev, st, GEMM_F32, v->xs, n_out, v->mm2, nullptr, d_out, nullptr, 1.0f));
     return htr_sync(dev);
 }
