@@ -10,13 +10,13 @@
 //             TM × TN v_mfma_f32_32x32x16_f16 tiles (lane layouts checked on the GPU: A lane ℓ holds
 //             A[ℓ%32][8(ℓ/32) …+7], B lane ℓ holds B[8(ℓ/32) …+7][ℓ%32], D lane ℓ register r is row 8(r/4) + 4(ℓ/32)
 //             + r%4, column ℓ%32). Tile shapes: 256 × 256 and 192 × 256 (8 waves of 128 × 64 / 96 × 64), 128 × 128
-//             (8 waves of 32 × 64; the FFN 4 of 64 × 64) and 64 × 64 (4 waves of 32 × 32); the launch takes the largest that still gives half a
-//             workgroup per CU, 192 rows where that takes fewer rows × rounds, and splits K for prompt-sized M.
+//             (8 waves of 32 × 64; the FFN 4 of 64 × 64) and 64 × 64 (4 waves of 32 × 32); the launch takes the largest
+//             that still gives half a workgroup per CU, 192 rows where that takes fewer rows × rounds, and splits K for prompt-sized M.
 //             The FFN's W tile is BN/2 gate rows and the same BN/2 up rows in alternating blocks of 32, so a wave's
 //             two column tiles are one gate and one up tile of the same outputs;
 //   K         through a ring of LDS stages filled by direct-to-LDS loads (global_load_lds_dwordx4): the 256-wide
-//             tiles and the FFN's 128-wide one in stages of 64 (a row's 128 bytes of the stage, whole cache lines) in a ring of 2, the stage
-//             after next loading while one is computed; the smaller tiles in stages of 32 in a ring of 4, the stage
+//             tiles and the FFN's 128-wide one in stages of 64 (a row's 128 bytes of the stage, whole cache lines) in a
+//             ring of 2, the stage after next loading while one is computed; the smaller tiles in stages of 32 in a ring of 4, the stage
 //             3 ahead loading. Inside a stage a row's 16-byte chunks sit XOR-placed (chunk ^ (row/4 % 4) for 4 a
 //             row, chunk ^ (row/2 % 8) for 8): 16 consecutive rows of one chunk fall on 16 different 16-byte bank
 //             groups (gfx950's LDS serves 16 lanes of a 16-byte read a cycle across 256 bytes);
@@ -521,6 +521,8 @@ int launch(htr_device *dev, hipStream_t st, int epi, GemmK &a, bool *normed = nu
         ((n_tiles[1] < want && a.k >= 1024) || (16 * n_tiles[1] <= 9 * dev->n_cu && a.k >= 4096))) {
         int sp = std::min(4, (dev->n_cu + n_tiles[1] - 1) / n_tiles[1]);
         while (sp > 1 && a.k % (32 * sp)) sp--;
+        // a graph of the caller's keeps no scratch address where the shape has another way
+        if (n_tiles[1] >= want && dev->capturing) sp = 1;
         if (sp > 1) {
             void *part = nullptr;
             HTR_TRY(htr_scratch(dev, SCR_GEMM_PART, (size_t)sp * a.m * a.rows[0] * 4, &part));
