@@ -615,8 +615,10 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
     // stage st in buffer b: its scores are in s; the next stage's are computed into sn under the softmax's VALU work
     auto step = [&](int st, int b, f32x16 &s, f32x16 &sn, auto mask) {
         constexpr bool MASK = decltype(mask)::value;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads of K stage st + 1 and V stage st
-        __builtin_amdgcn_s_barrier();                       // everyone's; K stage st and V stage st − 1 are read by all
+        // this wave's loads of K stage st + 1 and V stage st are in, its reads of K stage st and V stage st − 1 have
+        // their values (their MFMAs may stand behind the barrier); behind it everyone's, and the two buffers are free
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (st + 2 < n_stage) issue(st + 2, false);
         if (st + 1 < n_stage) issue(st + 1, true);
