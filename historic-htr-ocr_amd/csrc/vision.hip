@@ -313,8 +313,10 @@ __global__ __launch_bounds__(VW) void k_attn_vision(const float *Q, const _Float
         };
         static_assert(QG == 2 && AST == 2, "the turns of two groups, two blocks a stage");
         auto turn = [&](int st) {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads of stage st + 1
-            __builtin_amdgcn_s_barrier();                       // everyone's; and stage st − 1 is read by all
+            // this wave's loads of stage st + 1 are in and its reads of stage st − 1 have their values, wherever their
+            // MFMAs stand; behind the barrier everyone's
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             if (st + 2 < st1) issue(st + 2);
         };
@@ -339,7 +341,9 @@ __global__ __launch_bounds__(VW) void k_attn_vision(const float *Q, const _Float
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) pv(1, i);
-        __builtin_amdgcn_s_barrier();  // the next tile's first stage overwrites a buffer that another wave may still read
+        // the next tile's first stage overwrites a buffer that another wave may still read
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int g = 0; g < QG; g++) {
