@@ -458,9 +458,14 @@ __global__ __launch_bounds__(AW) void k_attn_decode(const float *q, const _Float
 // attention_causal.wgsl's arithmetic (text.rs:484-499; the same on every compute path): q·scale in f32, scores as
 // f32 dot products with the f16 keys, an online softmax in f32 over the keys each query sees (0 … its position),
 // out = acc · (1 / l). Here on the f16 matrix cores (v_mfma_f32_32x32x16_f16) with f32-grade operands: q·scale =
-// qh + ql and p·2^10 = ph + pl, each half rounded to f16 (the pair holds 22 bits; K and V are f16 already), so every
-// product is exact and every sum f32; the 2^10 (exact) keeps small p out of f16's subnormals and drops out with l,
-// which carries it too.
+// qh + ql and p·2^10 = ph + pl, each half rounded to f16 (K and V are f16 already), so every product of what is held is
+// exact and every sum f32; the 2^10 (exact) drops out with l, which carries it too. The p pair holds 22 bits of p down to
+// 2^-12 of a query's largest, and is within 2^-35 of that largest below (pl is subnormal there). The q pair holds 22 bits,
+// except that qh is rounded from the f32 product and ql is the rest beside the product rounded to f16 in one step (that
+// is how the compiler takes x·scale where both are wanted): where the f32 product is a tie the two f16 values differ, and
+// the pair is an f16 ulp off (5e-5 of random elements, none with a power of two as scale; the outputs' error against 64
+// bits is 4.8e-6 for it, 3e-7 without). Holding the product to one value would cost nothing, but moves single outputs by
+// up to 1e-3 of their size.
 //
 //   work     a workgroup takes 32 queries of both q heads of a KV head: 4 waves = 2 heads × the even / odd key blocks,
 //            the two parts merged through LDS at the end. A stage is 2 blocks of 32 keys (32 KB), K and V each

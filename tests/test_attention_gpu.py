@@ -160,15 +160,26 @@ def test_causal_attention_rejects_bad_ranges(dev):
         htr.causal_attention(dev, q, kc, vc, 1, 0, 6, 2, 8, 0.1, out)
 
 
+def _q_as_held(q, sc):
+    """the kernel's q·scale / scale in 64 bits: a pair of f16 values, the first rounded from the f32 product, the second
+    the rest beside the product rounded to f16 in one step. The two f16 roundings differ, by an ulp, where the f32 product
+    is a tie (5e-5 of random elements; never where scale is a power of two)"""
+    qs = (q * np.float32(sc)).astype(np.float32)
+    once = (q.astype(np.float64) * np.float64(np.float32(sc))).astype(np.float16)
+    lo = (qs - once.astype(np.float32)).astype(np.float16)
+    return (qs.astype(np.float16).astype(np.float64) + lo.astype(np.float64)) / np.float64(np.float32(sc))
+
+
+@pytest.mark.parametrize("sc", [0.125, float(np.float32(1 / np.sqrt(128)))])
 @pytest.mark.parametrize("n_q,pos0,n_kv,scale_q,off", [
     (31, 0, 1, 1.0, 0), (32, 31, 2, 1.0, 0), (65, 63, 3, 1.0, 0), (129, 1, 2, 1.0, 0), (7, 700, 2, 1.0, 0),
     (96, 32, 2, 40.0, 0),  # scores past 100: the running reference moves often, and far
     (40, 9, 2, 1.0, 1)])   # caches 2 bytes off a 16-byte boundary: copied before they are read
-def test_causal_attention_block_edges(dev, n_q, pos0, n_kv, scale_q, off):
-    """query and key counts around the blocks of 32 and the stages of 64 against fp64 softmax attention on the f16 keys,
-    row by row. Bar: q and p are held in 22 bits (2^-22 = 2.4e-7 a product) and a score's f32 sum of 128 products errs by
-    about 2^-24 of its magnitude, which the exponential turns into a relative error of p: 1e-5 up to scores of about 10,
-    times the scores' growth past that."""
+def test_causal_attention_block_edges(dev, n_q, pos0, n_kv, scale_q, off, sc):
+    """query and key counts around the blocks of 32 and the stages of 64 against fp64 softmax attention of the q that the
+    kernel holds on the f16 keys, row by row. Bar: q and p are held in 22 bits (2^-22 = 2.4e-7 a product) and a score's f32
+    sum of 128 products errs by about 2^-24 of its magnitude, which the exponential turns into a relative error of p: 1e-5
+    up to scores of about 10, times the scores' growth past that."""
     n_head, n_keys = 2 * n_kv, pos0 + n_q
     g = orc.Lcg(n_q * 11 + pos0)
     k = orc.f16_bits(g.f32(n_keys * n_kv * 128, 2.0)).reshape(n_keys, -1)
@@ -179,13 +190,13 @@ def test_causal_attention_block_edges(dev, n_q, pos0, n_kv, scale_q, off):
         raw = kv_head_major(a, n_kv).view(np.uint16).ravel()
         bufs.append(dev.upload(np.concatenate([np.zeros(off, np.uint16), raw, np.zeros(8 - off, np.uint16)])))
     out = dev.alloc(n_q * n_head * 128 * 4)
-    sc = 0.125  # exact in f32: q·scale is the same value however it is rounded to f16
     qb = dev.upload(q)
     rc = htr.lib().htr_causal_attention(dev.h, qb.ptr, bufs[0].ptr + 2 * off, bufs[1].ptr + 2 * off, n_q, pos0, n_head,
                                         n_kv, n_keys, sc, out.ptr)
     assert rc == 0, htr.last_error()
     got = out.download(np.float32).reshape(n_q, n_head * 128)
+    held = _q_as_held(q, sc)
     for t in range(n_q):
-        row = orc.attn_f64(q[t * n_head * 128:(t + 1) * n_head * 128], k, v, n_kv * 128, pos0 + t + 1, n_head, n_kv,
+        row = orc.attn_f64(held[t * n_head * 128:(t + 1) * n_head * 128], k, v, n_kv * 128, pos0 + t + 1, n_head, n_kv,
                            sc)
         assert rel_l2(got[t], row) < 1e-5 * max(1.0, scale_q / 4), t
