@@ -539,7 +539,7 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
     auto issue = [&](int st, bool isv) {
         const int s0 = CK * CKS * st;  // the stage's first key
         const char *base = (const char *)(isv ? vh : kh) + (size_t)s0 * (2 * D);
-        const uint32_t off = isv ? voff : koff, last = 2 * D * (n_keys - 1 - s0) + off;  // the last key's
+        const uint32_t off = isv ? voff : koff, last = 2 * D * min(n_keys - 1 - s0, CK * CKS - 1) + off;  // the last key's
 #pragma unroll
         for (int i = 0; i < 2 * CKS; i++)  // rows 16i + lrow of the stage: half a block
             lds_load16(base, min(2 * D * (16 * i + lrow) + off, last),

@@ -200,3 +200,20 @@ def test_causal_attention_block_edges(dev, n_q, pos0, n_kv, scale_q, off, sc):
         row = orc.attn_f64(held[t * n_head * 128:(t + 1) * n_head * 128], k, v, n_kv * 128, pos0 + t + 1, n_head, n_kv,
                            sc)
         assert rel_l2(got[t], row) < 1e-5 * max(1.0, scale_q / 4), t
+
+
+def test_causal_attention_past_four_gib_of_keys(dev):
+    """2^24 + 4 keys of one head (their bytes pass 32 bits): one query finds the key in row 10 among zeros, and nothing
+    else; the rows serve as values too. Bar: the zeros' sum of p is 16.8 million equal f32 terms, each added within 2^-24
+    of a sum that e^30 = 1e13 dwarfs; 1e-5 as in the other causal tests"""
+    n_keys, row = 2 ** 24 + 4, 10
+    kv = np.zeros((n_keys, 128), np.float16)
+    kv[row] = np.where(np.arange(128) % 2, 1.0, -1.0)
+    cache = dev.upload(kv)
+    q = np.concatenate([kv[row] * (s / 16.0) for s in (30.0, 40.0)]).astype(np.float32)  # scores 30 and 40 at scale 1/8
+    out = dev.alloc(2 * 128 * 4)
+    htr.causal_attention(dev, dev.upload(q), cache, cache, 1, n_keys - 1, 2, 1, n_keys, 0.125, out)
+    got = out.download(np.float32).reshape(2, 128)
+    for h, s in enumerate((30.0, 40.0)):
+        assert rel_l2(got[h], kv[row].astype(np.float64) / (1.0 + (n_keys - 1) * np.exp(-s))) < 1e-5
+    cache.free()
