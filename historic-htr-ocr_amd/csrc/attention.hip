@@ -480,7 +480,9 @@ __global__ __launch_bounds__(AW) void k_attn_decode(const float *q, const _Float
 //            8(i / 4) + 4h + i % 4 (i < 16); the max over a query's keys is one swap across lane bit 5;
 //   softmax  p = 2^(s·log2 e + nm), nm = 10 − log2 e · (the max when it was last moved): one fma and one v_exp_f32 a
 //            score, and nm is the only state, so its rounding cancels between p, l and O. nm moves (and O and l are
-//            rescaled) only when some p would pass 2^15, so most blocks skip the 64-register rescale;
+//            rescaled) only when some p would pass 2^15, so most blocks skip the 64-register rescale. nm holds scores of
+//            2^26 to within 4, and p to 2^14 with them; a wave with a query whose scores could be larger (Σ |q·scale| of
+//            a half row from 512 on, against f16 keys of 65504 at most) keeps the max itself and takes s − max first;
 //   values   Oᵀ (128 dims × 32 queries) += Vᵀ·(ph + pl)ᵀ: the Vᵀ operand by ds_read_b64_tr_b16 (16 lanes read 4 key
 //            rows × 16 dims and each gets one dim's 4 keys), the P operand straight from the lane's score registers.
 //
@@ -551,6 +553,7 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
 
     // q·scale as f16 pairs: B operand of step ks = dims 16ks + 8hf … + 7 of query c
     half8 qh[8], ql[8];
+    bool far;
     {
         const float *qrow = q + ((size_t)qi * n_head + h) * D + 8 * hf;
         float x[8][8];
@@ -581,6 +584,7 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
                     x[ks + 4][e] = y0 * t.y + y1 * t.x;
                 }
         }
+        float size = 0.0f;
 #pragma unroll
         for (int ks = 0; ks < 8; ks++)
 #pragma unroll
@@ -589,7 +593,9 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
                 const _Float16 hi = (_Float16)qs;
                 qh[ks][e] = hi;
                 ql[ks][e] = (_Float16)(qs - (float)hi);
+                size += fabsf(qs);
             }
+        far = __builtin_amdgcn_ballot_w64(!(size < 512.0f)) != 0;
     }
     // the lane's fragment slots in a block: K step ks (key c, dims 16ks + 8hf …); V tile t (16-lane group: dims
     // 32t + 16(ℓ/16 % 2) …, keys 4hf + (ℓ%16)/4 of each 8-key group)
@@ -606,7 +612,7 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int i = 0; i < 16; i++) o[t][i] = 0.0f;
-    float nm = 3.0e38f, l = 0.0f;
+    float nm = 3.0e38f, l = 0.0f;  // far: nm is −max
 
     auto scores = [&](f32x16 &s, int st) {
         const int4 *blk = s_kv[st & 1][kp];
@@ -618,8 +624,8 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
         }
     };
     // stage st in buffer b: its scores are in s; the next stage's are computed into sn under the softmax's VALU work
-    auto step = [&](int st, int b, f32x16 &s, f32x16 &sn, auto mask) {
-        constexpr bool MASK = decltype(mask)::value;
+    auto step = [&](int st, int b, f32x16 &s, f32x16 &sn, auto mask, auto is_far) {
+        constexpr bool MASK = decltype(mask)::value, FAR = decltype(is_far)::value;
         // this wave's loads of K stage st + 1 and V stage st are in, its reads of K stage st and V stage st − 1 have
         // their values (their MFMAs may stand behind the barrier); behind it everyone's, and the two buffers are free
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
@@ -635,13 +641,19 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
             mx = fmaxf(mx, s[i]);
         }
         mx = pair_max<32>(mx);
-        if (__builtin_amdgcn_ballot_w64(fmaf(mx, LOG2E, nm) > P_TOP)) {
-            const float to = fminf(nm, fmaf(-mx, LOG2E, P_SHIFT)), corr = __builtin_amdgcn_exp2f(to - nm);
+        if (__builtin_amdgcn_ballot_w64(FAR ? mx + nm > 0.0f : fmaf(mx, LOG2E, nm) > P_TOP)) {
+            const float to = fminf(nm, FAR ? -mx : fmaf(-mx, LOG2E, P_SHIFT));
+            const float corr = __builtin_amdgcn_exp2f(FAR ? (to - nm) * LOG2E : to - nm);
             nm = to;
             l *= corr;
 #pragma unroll
             for (int t = 0; t < 4; t++) o[t] *= corr;
         }
+        if (FAR) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) s[i] += nm;
+        }
+        const float add = FAR ? P_SHIFT : nm;
         // the order pinned: behind each score MFMA of the next stage its share of this stage's softmax (left to itself
         // the compiler issues the MFMAs back to back and the softmax behind them)
         // (past the last stage: scores of what the buffer holds, not used)
@@ -668,8 +680,8 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
             sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks], qh[ks], ks ? sn : f32x16{}, 0, 0, 0);
             if (ks + 3 < 8) a[ks + 3] = *reinterpret_cast<const half8 *>(kb + ka[ks + 3]);
             else v[ks - 5] = vread(ks - 5, 0);
-            const float2_t p = {__builtin_amdgcn_exp2f(fmaf(s[2 * ks], LOG2E, nm)),
-                                __builtin_amdgcn_exp2f(fmaf(s[2 * ks + 1], LOG2E, nm))};  // masked: 2^(−inf) = 0
+            const float2_t p = {__builtin_amdgcn_exp2f(fmaf(s[2 * ks], LOG2E, add)),
+                                __builtin_amdgcn_exp2f(fmaf(s[2 * ks + 1], LOG2E, add))};  // masked: 2^(−inf) = 0
             const half2_t hi = __builtin_convertvector(p, half2_t);
             __builtin_memcpy(&ph[ks], &hi, 4);
             asm volatile("" : "+v"(ph[ks]));  // holds the conversion here
@@ -707,12 +719,19 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
     f32x16 s0, s1;
     scores(s0, 0);
     int st = 0;
+    // (the two kinds of wave pass the same barriers, one a stage)
+    if (far) {
+        for (; st < n_stage; st++) {
+            step(st, st & 1, s0, s1, std::true_type{}, std::true_type{});
+            s0 = s1;
+        }
+    }
     for (; st + 1 < n_full; st += 2) {
-        step(st, 0, s0, s1, std::false_type{});
-        step(st + 1, 1, s1, s0, std::false_type{});
+        step(st, 0, s0, s1, std::false_type{}, std::false_type{});
+        step(st + 1, 1, s1, s0, std::false_type{}, std::false_type{});
     }
     for (; st < n_stage; st++) {
-        step(st, st & 1, s0, s1, std::true_type{});
+        step(st, st & 1, s0, s1, std::true_type{}, std::false_type{});
         s0 = s1;
     }
     l = pair_sum<32>(l);
@@ -732,8 +751,8 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
 #pragma unroll
     for (int p = 0; p < CKS; p++) top = fminf(top, s_ml[2 * p + hh][0][c]);
 #pragma unroll
-    for (int p = 0; p < CKS; p++) {
-        w[p] = __builtin_amdgcn_exp2f(top - s_ml[2 * p + hh][0][c]);  // a part without keys: 2^(−3e38) = 0
+    for (int p = 0; p < CKS; p++) {  // (both parts of a head hold the same queries: far or not alike)
+        w[p] = __builtin_amdgcn_exp2f((top - s_ml[2 * p + hh][0][c]) * (far ? LOG2E : 1.0f));  // a part without keys: 0
         lsum = fmaf(s_ml[2 * p + hh][1][c], w[p], lsum);
     }
     const float inv = 1.0f / lsum;

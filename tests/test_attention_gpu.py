@@ -217,3 +217,26 @@ def test_causal_attention_past_four_gib_of_keys(dev):
     for h, s in enumerate((30.0, 40.0)):
         assert rel_l2(got[h], kv[row].astype(np.float64) / (1.0 + (n_keys - 1) * np.exp(-s))) < 1e-5
     cache.free()
+
+
+@pytest.mark.parametrize("n_q,pos0", [(1, 0), (40, 70), (70, 300)])
+def test_causal_attention_of_scores_up_to_two_to_the_31(dev, n_q, pos0):
+    """scores from 1e3 to 2e9, exact in f32 (q and k multiples of one sign vector): the softmax is of the largest key, or
+    of several equal ones in equal parts, whatever the scores' size. f32 holds such scores 128 apart, so a reference of
+    the softmax that is rounded to f32 may be off by far more than f16's range of p. Rows of one workgroup differ in size"""
+    n_head, n_kv, n_keys = 2, 1, pos0 + n_q
+    rng = np.random.default_rng(n_q + pos0)
+    sign = np.where(np.arange(128) % 3, 1.0, -1.0)
+    c = rng.integers(-2000, 2001, n_keys)
+    c[rng.integers(0, n_keys, n_keys // 4)] = 2000  # equal largest keys
+    k = orc.f16_bits((c[:, None] * sign).astype(np.float32).ravel()).reshape(n_keys, 128)
+    v = orc.f16_bits(rng.standard_normal(n_keys * 128).astype(np.float32)).reshape(n_keys, 128)
+    t = 2.0 ** rng.choice([-4, 5, 13, 16], n_q * n_head)  # scores 16·c·t
+    q = (t[:, None] * sign).astype(np.float32)
+    out = dev.alloc(n_q * n_head * 128 * 4)
+    htr.causal_attention(dev, dev.upload(q), dev.upload(kv_head_major(k, 1)), dev.upload(kv_head_major(v, 1)), n_q, pos0,
+                         n_head, n_kv, n_keys, 0.125, out)
+    got = out.download(np.float32).reshape(n_q, n_head * 128)
+    for i in range(n_q):
+        row = orc.attn_f64(q[i * n_head:(i + 1) * n_head].ravel(), k, v, 128, pos0 + i + 1, n_head, n_kv, 0.125)
+        assert rel_l2(got[i], row) < 1e-5, i
