@@ -178,7 +178,8 @@ __global__ __launch_bounds__(VW) void k_heads_f16(const float *K, const float *V
 constexpr int FQ = 32, FB = 32, FWAVES = VW / 64, AST = 2;
 // p = 2^(s·log2 e + nm), nm = 10 − log2 e · (the max when it was last moved): nm moves, and O and l are rescaled, only
 // when some p would pass 2^15 (f16 holds 65504), so most blocks skip the rescale; nm is the only state, its rounding
-// cancels between p, l and O
+// cancels between p, l and O. That rounding is up to 4 at 2^26 and doubles with the max: from there on the shift is left
+// out, so p stays in f16's range up to 2^28, as far as e^(s − max) taken as 2^(s·log2 e − max·log2 e) did
 constexpr float P_SHIFT = 10.0f, P_TOP = 15.0f, LOG2E = 1.4426950408889634f;
 constexpr int RING = 3;      // stages in LDS: the one in use, the next one (its first K block), one loading
 constexpr int CUT_COST = 8;  // stages that a cut has to save: the partial sums' way through memory and the merge's launch
@@ -286,7 +287,8 @@ __global__ __launch_bounds__(VW) void k_attn_vision(const float *Q, const _Float
                 }
                 mx = pair_max<32>(mx);
                 if (__builtin_amdgcn_ballot_w64(fmaf(mx, LOG2E, nm[X]) > P_TOP)) {
-                    const float to = fminf(nm[X], fmaf(-mx, LOG2E, P_SHIFT)), corr = __builtin_amdgcn_exp2f(to - nm[X]);
+                    const float to = fminf(nm[X], fmaf(-mx, LOG2E, fabsf(mx) < 0x1p26f ? P_SHIFT : 0.0f));
+                    const float corr = __builtin_amdgcn_exp2f(to - nm[X]);
                     nm[X] = to;
                     l[X] *= corr;
 #pragma unroll

@@ -51,6 +51,28 @@ def test_tiny_encoder_on_cut_attention_tiles_matches_oracle(tiny, w, h):
     assert e < 2e-4  # the bar of the tiny encoders' first layer
 
 
+def test_encoder_keeps_scores_of_two_to_the_27(dev):
+    """a page of one colour, q = 8·k and k ~ 1300: every query's largest score is its own key's, 1.0e8 … 1.2e8 of the f32
+    values 8 apart, and every value row is the same, so the attention's output is that row whatever the softmax's weights
+    are, if they are finite"""
+    cfg = dict(tiny_vision_cfg(), image_size=1540)
+    t = tiny_vision_tensors(cfg)
+
+    def times(blocks, f):  # the blocks' scales times a power of two
+        b = blocks.reshape(-1, 34).copy()
+        b[:, :2] = (b[:, :2].copy().view(np.float16) * np.float16(f)).view(np.uint8)
+        return b.reshape(-1)
+
+    k = t["layers"][0]["k"]
+    t["layers"][0] = dict(t["layers"][0], q=times(k, 16384), k=times(k, 2048))
+    v = htr.Vision(dev, cfg, t)
+    for colour in ((255, 255, 255), (200, 30, 90), (0, 0, 0)):
+        rgb = np.ascontiguousarray(np.broadcast_to(np.array(colour, np.uint8), (140, 112, 3)))
+        e = rel_l2(v.encode(rgb, 1), orc.vision_encode(cfg, t, rgb, 1))
+        assert e < 2e-4, colour  # the bar of the tiny encoders' first layer
+    v.free()
+
+
 def test_encoder_rejects_unbaked_pages(tiny):
     cfg, t, v = tiny
     with pytest.raises(htr.HtrError, match="not baked"):
