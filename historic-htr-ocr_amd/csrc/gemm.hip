@@ -40,8 +40,11 @@ __global__ __launch_bounds__(256) void k_swiglu(float *g, const float *u, size_t
 //   F32 path  every product of the exact q8_0 value with the f32 X. A quant is a bf16 value (7 bits) and X is the sum
 //             of three (EX: its top 8 bits, the next 8, the last 8, each truncated, so x = b1 + b2 + b3 exactly), so
 //             three bf16 MFMAs add a block's Σ q·x in f32 with every product exact, and one f32 fma per output and
-//             block adds d·Σ q·x: three 16-bit MFMAs stand for what takes f32 ones sixteen times as long. Exact for
-//             |x| < 2^115 (a block's sum of q·x stays finite where the scaled one does); ±inf and NaN pass as they are.
+//             block adds d·Σ q·x: three 16-bit MFMAs stand for what takes f32 ones sixteen times as long. That holds for
+//             a tile without |x| from 2^115 on (a block's sum of q·x may overflow where the scaled one does not), without
+//             bits of an x under bf16's smallest and without an infinite scale; one that meets them is done again by
+//             wide_blocks. Looking for them costs nothing measurable; splitting and scaling every tile that way instead
+//             12 % (1023 × 1024 × 3072 onto the residual 36.1 → 40.6 µs).
 // Work: a workgroup owns 64T × 64T outputs; KG groups of 4 waves (2 × 2, 32T × 32T outputs a wave) take the K stages in
 // turn, each through its own pair of LDS buffers, and their sums are added in group order through LDS at the end: a
 // prompt of some hundred rows makes few tiles, and the groups give such a CU four waves a SIMD to hide the loads'
@@ -51,7 +54,7 @@ __global__ __launch_bounds__(256) void k_swiglu(float *g, const float *u, size_t
 // Bound: the 128 × 128 tile's MFMAs and conversions about even; the 64 × 64 ones by the stages' load latency. Measured
 // against the kernels before it (f32 FMA tiles on the f16 path, v_mfma_f32_32x32x2_f32 on the F32 path), a call: f16
 // 48 × 1024 × 2048 231 → 13.4 µs, 1925 × 3072 × 1024 422 → 30.4 µs (399 TFLOP/s); F32 1023 × 1024 × 3072 onto the
-// residual 111 → 36 µs (179 TFLOP/s, past the f32 MFMA's 157 peak). Error against 64 bits 5.6e-7 … 9.8e-7 → 1.2e-7 …
+// residual 111 → 35 µs (185 TFLOP/s, past the f32 MFMA's 157 peak). Error against 64 bits 5.6e-7 … 9.8e-7 → 1.2e-7 …
 // 2.0e-7: a block's 96 products are summed inside the matrix unit before the one f32 fma that scales them.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -69,31 +72,86 @@ __device__ __forceinline__ uint32_t hi_pair(uint32_t a, uint32_t b) { return __b
 
 __device__ __forceinline__ int8_t q_byte(int2 v, int e) { return (int8_t)((uint32_t)(e < 4 ? v.x : v.y) >> (8 * (e & 3))); }
 
+__device__ __forceinline__ int4 hi_halves(const uint32_t (&b)[8]) {
+    return make_int4((int)hi_pair(b[0], b[1]), (int)hi_pair(b[2], b[3]), (int)hi_pair(b[4], b[5]), (int)hi_pair(b[6], b[7]));
+}
+
+// what a tile has met of X and of the scales: the largest magnitude that is not a NaN, and what the third pieces left over
+struct Q8Seen {
+    float top = 0.0f;
+    uint32_t rest = 0;
+    __device__ __forceinline__ void add(float a, float b) {
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(top) : "v"(a), "v"(b));
+    }
+    __device__ __forceinline__ bool wide() const { return !(top < 0x1p115f) || (rest & 0xffffu); }
+};
+
 // 8 values as three bf16 pieces, x = b1 + b2 + b3: each piece the top 16 bits of what is left (no rounding: 24 = 3 · 8
-// bits). ±inf and NaN: the value itself and two zeros (inf − inf would make NaN of an infinity)
-__device__ __forceinline__ void split3(const float (&x)[8], int4 (&out)[3]) {
+// bits). Nothing is left over from |x| = 2^-110 on (bf16 ends at 2^-133). NaN: a NaN, at least in the second piece
+__device__ __forceinline__ void split3(const float (&x)[8], int4 (&out)[3], Q8Seen &seen) {
     uint32_t b[3][8];
-    bool odd = false;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
         b[0][e] = __float_as_uint(x[e]);
         const float r1 = x[e] - __uint_as_float(b[0][e] & 0xffff0000u);
         b[1][e] = __float_as_uint(r1);
         b[2][e] = __float_as_uint(r1 - __uint_as_float(b[1][e] & 0xffff0000u));
-        odd |= !(fabsf(x[e]) <= 3.4028235e38f);
+        seen.rest |= b[2][e];
+        if (e & 1) seen.add(x[e - 1], x[e]);
     }
-    if (__builtin_expect(odd, 0)) {
 #pragma unroll
-        for (int e = 0; e < 8; e++)
-            if (!(fabsf(x[e]) <= 3.4028235e38f)) {
-                if (x[e] != x[e]) b[0][e] |= 0x00400000u;  // a NaN whose payload sits in the low half stays one
-                b[1][e] = b[2][e] = 0u;
+    for (int s = 0; s < 3; s++) out[s] = hi_halves(b[s]);
+}
+
+// 32 × 32 outputs of a wave over the blocks b0, b0 + step, … below b1, each product exact for all of f32 and a block's sum
+// finite where the scaled one is: x = b1 + 2^-8·b2 + 2^-16·b3, what is left scaled up each time (it is under 2^-7·|x|), so
+// that nothing is lost at the lower end, against the quants with 2^0, 2^-8 and 2^-16; and d = 2^e · m, with 2^e on the
+// quants (q · 2^e is a bf16 value) and m = 1 … 2, with d's sign, on the block's sum. ±inf, NaN, d = ±inf and NaN as the
+// products q·d·x give them. The products and their order are those of the caller's own pass (ko, kh: where the lane's first
+// 8 k of a block start, and its other 8), so a row's results do not depend on the other rows. Straight from memory, one
+// block at a time: a tile that needs it takes several times as long
+__device__ __forceinline__ f32x16 wide_blocks(const float *x, const int8_t *q, const _Float16 *d, int b0, int b1, int step,
+                                              int ko, int kh) {
+    typedef uint16_t ushort8 __attribute__((ext_vector_type(8)));
+    f32x16 c = {};
+#pragma unroll 1
+    for (int b = b0; b < b1; b += step) {
+        const float ds = (float)d[b];
+        const float pow2 = fmaxf(__uint_as_float(__float_as_uint(ds) & 0x7f800000u), 0x1p-24f);  // of 0: m is 0
+        const float mant = __uint_as_float((__float_as_uint(ds) & 0x807fffffu) | 0x3f800000u);
+        f32x16 p = {};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int at = 32 * b + ko + h * kh;
+            uint32_t f[3][8], w[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float v = x[at + e], r1 = (v - __uint_as_float(__float_as_uint(v) & 0xffff0000u)) * 256.0f;
+                const float r2 = (r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u)) * 256.0f;
+                const bool inf = fabsf(v) == INFINITY;  // inf − inf would make NaN of it
+                f[0][e] = __float_as_uint(v);
+                f[1][e] = inf ? 0u : __float_as_uint(r1);
+                f[2][e] = inf ? 0u : __float_as_uint(r2);
+                w[e] = __float_as_uint((float)q[at + e] * pow2);
             }
-    }
+            ushort8 wb;
+            const int4 w4 = hi_halves(w);
+            __builtin_memcpy(&wb, &w4, 16);
 #pragma unroll
-    for (int s = 0; s < 3; s++)
-        out[s] = make_int4((int)hi_pair(b[s][0], b[s][1]), (int)hi_pair(b[s][2], b[s][3]),
-                           (int)hi_pair(b[s][4], b[s][5]), (int)hi_pair(b[s][6], b[s][7]));
+            for (int pl = 0; pl < 3; pl++) {
+                if (pl) wb = __builtin_elementwise_sub_sat(wb, (ushort8)(uint16_t)(8 << 7));  // 8 off each exponent; a 0 stays
+                const int4 a4 = hi_halves(f[pl]);
+                bf16x8 a, wp;
+                __builtin_memcpy(&a, &a4, 16);
+                __builtin_memcpy(&wp, &wb, 16);
+                p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wp, p, 0, 0, 0);
+            }
+        }
+        const float m = ds == 0.0f || ds != ds ? ds : mant;
+#pragma unroll
+        for (int i = 0; i < 16; i++) c[i] = fmaf(p[i], m, c[i]);
+    }
+    return c;
 }
 
 template <bool EX, int T, int KG> struct Q8Tile {
@@ -112,6 +170,7 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const in
     constexpr int KB = C::KB, CPR = C::CPR, R = C::R, UN = C::UN;
     __shared__ __attribute__((aligned(16))) int4 s_t[C::LDS];
     __shared__ float s_d[EX ? KG : 1][2][EX ? C::BT : 1];
+    __shared__ int s_wide;
     const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8), tid = threadIdx.x & 255, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
     // workgroup b runs on XCD b mod 8: each XCD takes a contiguous band of tiles, walked 4 tile rows at a time, so the
@@ -150,6 +209,7 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const in
             r.d[i] = wd[wr * nb + b];
         }
     };
+    Q8Seen seen;
     auto lstore = [&](const Regs &r, int st, int buf) {
         int4 *s = buf0 + buf * C::BUF;
 #pragma unroll
@@ -166,14 +226,14 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const in
             }
             if constexpr (EX) {
                 int4 p[3];
-                split3(v, p);
+                split3(v, p, seen);
+                seen.add(d, 0.0f);
 #pragma unroll
                 for (int t = 0; t < 3; t++) s[t * C::BT * CPR + at] = p[t];
                 uint32_t f[8];
 #pragma unroll
                 for (int e = 0; e < 8; e++) f[e] = __float_as_uint((float)q_byte(r.q[i], e));
-                s[C::ACH + at] = make_int4((int)hi_pair(f[0], f[1]), (int)hi_pair(f[2], f[3]),
-                                           (int)hi_pair(f[4], f[5]), (int)hi_pair(f[6], f[7]));
+                s[C::ACH + at] = hi_halves(f);
                 if (c == 0) s_d[grp][buf][rr] = d;
             } else {
                 half2_t hx[4], hw[4];
@@ -255,6 +315,7 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const in
     // group grp's stage i is grp + KG·i; every group runs the same count (a stage past the last is zeros). Step i reads
     // buffer i % 2 while stage i + 1 is stored to the other, which step i − 1 read before the barrier that ended it
     const int steps = (nst + KG - 1) / KG;
+    if (EX && threadIdx.x == 0) s_wide = 0;  // before the first barrier
 #pragma unroll
     for (int r = 0; r < R; r++) gload(ring[r], grp + KG * r);
     lstore(ring[0], grp, 0);
@@ -270,6 +331,19 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const in
                 gload(ring[(r + 1) % R], grp + KG * (i + 1 + R));
                 lds_barrier();
             }
+        }
+    }
+    if constexpr (EX) {
+        if (__builtin_amdgcn_ballot_w64(seen.wide()) && lane == 0) s_wide = 1;
+        __syncthreads();
+        if (__builtin_expect(s_wide, 0)) {
+#pragma unroll
+            for (int i = 0; i < T; i++)
+#pragma unroll
+                for (int j = 0; j < T; j++) {
+                    const size_t xr = min(row0 + fa + 32 * i, m - 1), wr = min(col0 + fb + 32 * j, n - 1);
+                    c[i][j] = wide_blocks(x + xr * k, wq + wr * k, wd + wr * nb, grp, nb, KG, 8 * hk, 16);
+                }
         }
     }
     // lane ℓ, register r: row 8(r/4) + 4(ℓ/32) + r%4, column ℓ%32 of each 32 × 32 tile
@@ -362,6 +436,7 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void k_gemm_q8_0_few(const float *x
         r.d = d[b];
     };
     f32x16 c = {};
+    Q8Seen seen;
     auto use = [&](const Regs &r) {
         const int2 qs[2] = {make_int2(r.q.x, r.q.y), make_int2(r.q.z, r.q.w)};
         if constexpr (EX) {
@@ -371,8 +446,7 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void k_gemm_q8_0_few(const float *x
                 uint32_t f[8];
 #pragma unroll
                 for (int e = 0; e < 8; e++) f[e] = __float_as_uint((float)q_byte(qs[h], e));
-                const int4 v = make_int4((int)hi_pair(f[0], f[1]), (int)hi_pair(f[2], f[3]), (int)hi_pair(f[4], f[5]),
-                                         (int)hi_pair(f[6], f[7]));
+                const int4 v = hi_halves(f);
                 __builtin_memcpy(&b[h], &v, 16);
             }
             f32x16 p;
@@ -381,7 +455,7 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void k_gemm_q8_0_few(const float *x
                 const float4 u = r.a[2 * h], v = r.a[2 * h + 1];
                 const float f[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
                 int4 a[3];
-                split3(f, a);
+                split3(f, a, seen);
 #pragma unroll
                 for (int pl = 0; pl < 3; pl++) {
                     bf16x8 av;
@@ -391,6 +465,7 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void k_gemm_q8_0_few(const float *x
             }
 #pragma unroll
             for (int i = 0; i < 16; i++) c[i] = fmaf(p[i], (float)r.d, c[i]);
+            seen.add((float)r.d, 0.0f);
         } else {
             const float ds = (float)r.d;
 #pragma unroll
@@ -423,6 +498,8 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void k_gemm_q8_0_few(const float *x
                 gload(ring[i], i0 + i + FEW_R);
             }
     }
+    if (EX && __builtin_expect(__builtin_amdgcn_ballot_w64(seen.wide()) != 0, 0))
+        c = wide_blocks(xr, q, d, b0, b1, 1, 0, 8);  // (xr and q start at the lane's half of a block)
     // lane ℓ, register r: row 8(r/4) + 4(ℓ/32) + r%4, column ℓ%32
 #pragma unroll
     for (int i = 0; i < 16; i++) s_o[wave][8 * (i >> 2) + 4 * hk + (i & 3)][r32] = c[i];

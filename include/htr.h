@@ -190,7 +190,8 @@ int htr_choose_many(htr_device *dev, float *d_logits, int n_vocab, int n, uint32
                     int window, float rp, uint32_t *d_tok);
 
 /* Y[m][N] (+= with acc) X·Wᵀ, X f32 [m][K], W q8_0 [N][K] (gpu.rs:1963-2014 Batch::matmul with a q8_0 weight, the
- * prefill's GEMMs): on the device's compute path — F32: exact dequant, f32 fma (matmul128_q8_0 / matmul.wgsl);
+ * prefill's GEMMs): on the device's compute path — F32: exact dequant, f32 sums over all of f32's range
+ * (matmul128_q8_0 / matmul.wgsl);
  * F16: X and W rounded to f16 as they enter the tiles, f32 sums (matmul128h_q8_0 / matmul_coop_q8_0). Any shape
  * (K a multiple of 32). */
 int htr_matmul_q8_0(htr_device *dev, const float *d_x, size_t m, const htr_weight *w, float *d_y, int acc);

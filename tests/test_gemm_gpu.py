@@ -279,14 +279,14 @@ def test_matmul_q8_0_few_rows_against_fp64(dev, m, n, k, off):
 
 def test_matmul_q8_0_f32_path_keeps_infinities_and_nans(dev):
     """one infinity a row gives ±inf (NaN where its quant is 0), a NaN a NaN — also one whose payload is in its low
-    half — and the largest finite values stay exact; the other rows are untouched"""
+    half — and the largest finite value stays one; the other rows are untouched"""
     m, n, k = 6, 70, 128
     blocks = htr.synth_q8_0(77, n, k).reshape(n, k // 32, 34).copy()
     blocks[5, 1, 2 + 3] = 0  # the quant of k = 35 in row 5
     x = htr.synth_normal(78, m * k).reshape(m, k)
     x[0, 35], x[1, 35], x[2, 64] = np.inf, -np.inf, np.nan
     x[3, 7] = np.array([0x7F800001], np.uint32).view(np.float32)[0]
-    x[4, 100] = np.float32(2.0 ** 100)
+    x[4, 100] = np.finfo(np.float32).max
     w, xb = htr.Weight(dev, blocks.reshape(-1), n, k), dev.upload(x)
     y, keep = dev.alloc(m * n * 4), dev.compute
     try:
@@ -302,6 +302,46 @@ def test_matmul_q8_0_f32_path_keeps_infinities_and_nans(dev):
     assert np.isnan(got[2:4]).all() and np.isnan(got[0, 5]) and np.isinf(got[0, 6])
     assert np.array_equal(np.sign(got[np.isinf(got)]), np.sign(want[np.isinf(want)]))
     np.testing.assert_allclose(got[ok], want[ok], rtol=1e-4, atol=1e-4)
+    w.free()
+
+
+# the few-row kernel and each tile of the other one
+@pytest.mark.parametrize("m,n,k", [(12, 65, 96), (32, 1000, 96), (65, 70, 160), (333, 3072, 64), (2050, 2049, 64)])
+def test_matmul_q8_0_f32_path_over_the_range_of_f32(dev, m, n, k):
+    """rows of X from subnormal to the largest finite values, on weights of any scale (subnormal f16, both signs, 0, three
+    infinite or NaN): within the f32 rounding of the sum's own terms wherever these stay in f32's range, at both of its ends. A product or sum
+    under f32's smallest normal value is a multiple of 2^-149, which the terms' count of half steps allows for"""
+    rng = np.random.default_rng(m + n)
+    blocks = htr.synth_q8_0(3 * m + n, n, k).reshape(n, k // 32, 34).copy()
+    scale = (rng.choice([2.0 ** -24 * 3, 2.0 ** -16, -2.0 ** -12, 2.0 ** -7, 1.0, -60000.0, 0.0], (n, k // 32, 1))
+             * rng.uniform(0.5, 1.0, (n, k // 32, 1))).astype(np.float16)
+    scale[5, 1], scale[7, 0], scale[9, 1] = np.inf, -np.inf, np.nan
+    blocks[5, 1, 2:] = blocks[7, 0, 2:] = 3  # with a row of one sign: the infinity, with the others inf − inf
+    blocks[:, :, :2] = scale.view(np.uint8)
+    ex = np.array([127, 126, 119, 116, 112, 60, 0, -100, -110, -114, -118, -122, -126, -134, -142])[np.arange(m) % 15]
+    x = np.ldexp(rng.uniform(1.0, 2.0, (m, k)) * rng.choice([-1, 1], (m, k)), ex[:, None]).astype(np.float32)
+    x[6] = np.abs(x[6])
+    w, w64, keep = htr.Weight(dev, blocks.reshape(-1), n, k), _deq64(blocks.reshape(-1), n, k), dev.compute
+    y = dev.alloc(m * n * 4)
+    try:
+        dev.compute = htr.COMPUTE_F32
+        htr.matmul_q8_0(dev, dev.upload(x), m, w, y)
+    finally:
+        dev.compute = keep
+    got, x64 = y.download(np.float32).reshape(m, n).astype(np.float64), x.astype(np.float64)
+    size, terms = np.abs(x64) @ np.abs(w64).T, k // 32 + 98
+    inside = size < 2.0 ** 127
+    assert inside[ex == 127].any() and np.delete(inside, (5, 7, 9), axis=1)[ex < 100].all()
+    with np.errstate(invalid="ignore"):
+        want = x64 @ w64.T
+        err = np.abs(got - want)
+    odd = got[ex < 100][:, [5, 7, 9]], want[ex < 100][:, [5, 7, 9]]  # infinite and NaN scales
+    assert not np.isfinite(odd[1]).any() and np.isinf(odd[1]).any()
+    assert np.array_equal(odd[0], odd[1], equal_nan=True)
+    bound = terms * (2.0 ** -24 * size + 2.0 ** -150)
+    assert np.all(err[inside] <= bound[inside]), [(int(e), float(np.max((err / bound)[(ex == e)[:, None] & inside])))
+                                                  for e in np.unique(ex)]
+    y.free()
     w.free()
 
 
