@@ -116,5 +116,6 @@ template <int N> __device__ __forceinline__ float wave_sum_rows(float (&v)[N], i
 // the builtin the compiler makes the next LDS read wait for every load in flight (vmcnt 0), which it cannot tell apart
 // from the other buffer's; the asm writes no register, and the kernel waits for a stage's loads itself
 __device__ __forceinline__ void lds_load16(const void *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+                 : "memory", "m0");
 }

@@ -109,3 +109,17 @@ def test_no_lds_access_in_flight_at_a_barrier(tmp_path, source, kernels):
         seen += len(at)
         assert not any(at.values()), (name, sorted(at.items()))
     assert seen
+
+
+def test_inline_assembly_names_the_m0_it_writes():
+    """an asm statement that writes m0 lists it as clobbered: the compiler may hold a value of its own there"""
+    seen = 0
+    for path in sorted(os.listdir(os.path.join(PKG, "csrc"))):
+        with open(os.path.join(PKG, "csrc", path)) as f:
+            text = f.read()
+        for stmt in re.findall(r"\basm(?:__)?\s*(?:volatile)?\s*\((.*?)\);", text, re.S):
+            code, *operands = re.split(r'"\s*:', stmt, maxsplit=1)
+            if re.search(r"\bm0\s*,", code):
+                seen += 1
+                assert operands and '"m0"' in operands[0].split(":")[-1], (path, stmt)
+    assert seen
