@@ -72,7 +72,6 @@ enum {
     SCR_CAUSAL_KV = 4,  // aligned copies of caches that are not
     SCR_GEMM_PART = 5,  // split-K products [split][M][N]
     SCR_HANDOVER = 6,   // htr_debug_handover's words
-    SCR_VISION_PART = 7,  // the vision attention's sums of tiles cut along their keys
 };
 // the device's scratch buffer `slot` with at least `bytes` bytes (a larger one replaces it: the tickets' and best
 // keys' slots zero-filled, the others as htr_dev_alloc fills)
@@ -268,8 +267,10 @@ int launch_rms_norm_f16(htr_device *dev, hipStream_t st, const float *x, const f
 int launch_heads_f16(htr_device *dev, hipStream_t st, const float *k, const float *v, _Float16 *kv, int n_tok,
                      int n_head, const float *cs, int px, int max_pos);
 size_t vision_kv_bytes(int n_tok, int n_head);
+// part: vision_part_bytes of device memory for the sums of the tiles that are cut along their keys (0 bytes: none are)
+size_t vision_part_bytes(const htr_device *dev, int n_tok, int n_head);
 int launch_attn_vision(htr_device *dev, hipStream_t st, const float *q, const _Float16 *kv, _Float16 *o, int n_tok,
-                       int n_head, float scale, const float *cs, int px, int max_pos);
+                       int n_head, float scale, const float *cs, int px, int max_pos, float *part);
 // x (or gelu(x)) f32 [m][k] → f16 rows of nseg segments of kp values: hi = f16(x), or lo = f16(x − hi) in the segments of
 // lo_mask
 int launch_split_f16(htr_device *dev, hipStream_t st, const float *x, int m, int k, int kp, int nseg, int lo_mask,

@@ -188,11 +188,13 @@ struct VSplit {
     int groups, workers;      // groups of heads; workers a group
     int tiles, full;          // tiles a group; the first `full` of them are taken whole
     int n_qt, n_stage;        // tiles a head; stages of AST key blocks
+    __host__ __device__ int slots() const { return workers + tiles - full - 1; }  // a group's
     __host__ __device__ int first(int i) const {  // the first of worker i's stages of the tiles that are cut
         return (int)((long long)(tiles - full) * n_stage * i / workers);
     }
 };
-// a worker's sums of a part of a tile: [wave][query group][dim tile][16] registers, then nm and l, × 64 lanes
+// a worker's sums of a part of a tile: [wave][query group][dim tile][16] registers, then nm and l, × 64 lanes. Worker i's
+// part of cut tile t is the group's slot i + t (along the keys i or t grows from one part to the next)
 template <int QG> constexpr int PART = FWAVES * QG * 34 * 64;
 
 // QG groups of 32 queries a wave: the groups share every K / V fragment read from LDS and give the wave QG
@@ -379,7 +381,7 @@ __global__ __launch_bounds__(VW) void k_attn_vision(const float *Q, const _Float
         const int base = (t0 + u) * sp.n_stage;
         const bool part_of = u < cut;
         run(part_of ? sp.full + t0 + u : wk + (u - cut) * sp.workers, part_of ? max(a - base, 0) : 0,
-            part_of ? min(b - base, sp.n_stage) : sp.n_stage, part_of ? 2 * (grp * sp.workers + wk) + u : -1);
+            part_of ? min(b - base, sp.n_stage) : sp.n_stage, part_of ? grp * sp.slots() + wk + t0 + u : -1);
     }
 }
 
@@ -398,8 +400,7 @@ __global__ __launch_bounds__(64) void k_attn_vision_merge(const float *part, _Fl
     float nm = 3.0e38f, l = 0.0f, o[8] = {};
     for (int w = w0; w < sp.workers && sp.first(w) < base + sp.n_stage; w++) {
         if (sp.first(w + 1) == sp.first(w)) continue;
-        const int u = t - sp.first(w) / sp.n_stage;
-        const float *p = part + (size_t)(2 * (grp * sp.workers + w) + u) * PART<QG> + (size_t)wg * 34 * 64 + lane;
+        const float *p = part + (size_t)(grp * sp.slots() + w + t) * PART<QG> + (size_t)wg * 34 * 64 + lane;
         const float pn = p[32 * 64], pl = p[33 * 64];
         float v[8];
 #pragma unroll
@@ -527,33 +528,40 @@ int launch_heads_f16(htr_device *dev, hipStream_t st, const float *k, const floa
 
 size_t vision_kv_bytes(int n_tok, int n_head) { return (size_t)n_head * ((n_tok + FB - 1) / FB) * KVB; }
 
-int launch_attn_vision(htr_device *dev, hipStream_t st, const float *q, const _Float16 *kv, _Float16 *o, int n_tok,
-                       int n_head, float scale, const float *cs, int px, int max_pos) {
-    if (n_tok < 1) return htr_fail("vision attention: %d tokens", n_tok);
-    if (px < 1 || (n_tok + px - 1) / px > max_pos || px > max_pos)
-        return htr_fail("vision attention: %d tokens on %d columns, rope table of %d positions", n_tok, px, max_pos);
-    // two query groups a wave: 0.69 ms a layer at 12100 patches against 0.79 ms with one (223 VGPRs, 2 waves a SIMD;
-    // forcing 3 spills 111 of them)
-    constexpr int QG = 2;
-    const int n_blk = (n_tok + FB - 1) / FB;
+// two query groups a wave: 0.69 ms a layer at 12100 patches against 0.79 ms with one (223 VGPRs, 2 waves a SIMD; forcing 3
+// spills 111 of them)
+constexpr int VQG = 2;
+
+static VSplit vision_split(const htr_device *dev, int n_tok, int n_head) {
     VSplit sp{};
     sp.groups = n_head % 8 == 0 ? 8 : 1;
     sp.workers = 2 * dev->n_cu / sp.groups;
-    sp.n_qt = (n_tok + QG * FQ * FWAVES - 1) / (QG * FQ * FWAVES);
-    sp.n_stage = (n_blk + AST - 1) / AST;
+    sp.n_qt = (n_tok + VQG * FQ * FWAVES - 1) / (VQG * FQ * FWAVES);
+    sp.n_stage = ((n_tok + FB - 1) / FB + AST - 1) / AST;
     sp.tiles = n_head / sp.groups * sp.n_qt;
     sp.full = sp.tiles;
     // the tiles past the full rounds are cut where that shortens the last round by more than the merge costs
     const int left = sp.tiles % sp.workers;
     if (left && (left * sp.n_stage + sp.workers - 1) / sp.workers + CUT_COST < sp.n_stage) sp.full -= left;
-    float *part = nullptr;
-    if (sp.full < sp.tiles)
-        HTR_TRY(htr_scratch(dev, SCR_VISION_PART, (size_t)2 * sp.groups * sp.workers * PART<QG> * 4, (void **)&part));
-    hipLaunchKernelGGL(k_attn_vision<QG>, dim3(sp.groups * sp.workers), dim3(VW), 0, st, q, kv, o, n_tok, n_head, n_blk, sp,
-                       scale, cs, px, max_pos, part);
+    return sp;
+}
+
+size_t vision_part_bytes(const htr_device *dev, int n_tok, int n_head) {
+    const VSplit sp = vision_split(dev, n_tok, n_head);
+    return sp.full == sp.tiles ? 0 : (size_t)sp.groups * sp.slots() * PART<VQG> * sizeof(float);
+}
+
+int launch_attn_vision(htr_device *dev, hipStream_t st, const float *q, const _Float16 *kv, _Float16 *o, int n_tok,
+                       int n_head, float scale, const float *cs, int px, int max_pos, float *part) {
+    if (n_tok < 1) return htr_fail("vision attention: %d tokens", n_tok);
+    if (px < 1 || (n_tok + px - 1) / px > max_pos || px > max_pos)
+        return htr_fail("vision attention: %d tokens on %d columns, rope table of %d positions", n_tok, px, max_pos);
+    const VSplit sp = vision_split(dev, n_tok, n_head);
+    hipLaunchKernelGGL(k_attn_vision<VQG>, dim3(sp.groups * sp.workers), dim3(VW), 0, st, q, kv, o, n_tok, n_head,
+                       (n_tok + FB - 1) / FB, sp, scale, cs, px, max_pos, part);
     HTR_TRY(htr_launched(dev, "k_attn_vision"));
     if (sp.full == sp.tiles) return 0;
-    hipLaunchKernelGGL(k_attn_vision_merge<QG>, dim3(sp.groups * (sp.tiles - sp.full), 16 * QG), dim3(64), 0, st, part, o,
+    hipLaunchKernelGGL(k_attn_vision_merge<VQG>, dim3(sp.groups * (sp.tiles - sp.full), 16 * VQG), dim3(64), 0, st, part, o,
                        n_tok, n_head, sp);
     return htr_launched(dev, "k_attn_vision_merge");
 }

@@ -50,6 +50,8 @@ struct htr_vision {
     uint8_t *rgb = nullptr;
     size_t rgb_cap = 0;
     float *x = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *tmp = nullptr, *cs = nullptr;
+    float *part = nullptr;  // the attention's parts of cut tiles (not every page has them, and more patches may need less)
+    size_t part_cap = 0;
     _Float16 *h16 = nullptr, *a16 = nullptr, *g16 = nullptr, *kv = nullptr;
     // the f32 operands of the patch embedding and the projector as f16 pieces (k_split_f16): the patch embedding
     // weight [dim][hi | lo | hi] in segments of pe_kp (the patch's 3·p² values padded to a multiple of 32); the
@@ -113,13 +115,15 @@ int split_patch_embd(htr_vision *v, size_t pp) {
 
 void free_bufs(htr_vision *v) {
     for (void *p : {(void *)v->rgb, (void *)v->x, (void *)v->q, (void *)v->k, (void *)v->v, (void *)v->tmp,
-                    (void *)v->cs, (void *)v->h16, (void *)v->a16, (void *)v->g16, (void *)v->kv, (void *)v->xs})
+                    (void *)v->cs, (void *)v->h16, (void *)v->a16, (void *)v->g16, (void *)v->kv, (void *)v->xs,
+                    (void *)v->part})
         if (p) htr_dev_free(v->dev, p);
     v->rgb = nullptr;
     v->x = v->q = v->k = v->v = v->tmp = v->cs = nullptr;
     v->h16 = v->a16 = v->g16 = v->kv = v->xs = nullptr;
+    v->part = nullptr;
     v->n_cap = v->pos_cap = 0;
-    v->rgb_cap = 0;
+    v->rgb_cap = v->part_cap = 0;
 }
 
 // buffers for n patches (and the projector: merged n/4·dim, mm.1 n/4·proj_dim fit in k / v)
@@ -153,6 +157,14 @@ int ensure_bufs(htr_vision *v, int n, int max_pos, size_t rgb_bytes) {
         v->n_cap = n;
         v->pos_cap = max_pos;
         v->rgb_cap = rgb_bytes;
+    }
+    const size_t part = vision_part_bytes(dev, n, c.n_head);
+    if (part > v->part_cap) {
+        if (v->part) htr_dev_free(dev, v->part);
+        v->part = nullptr;
+        v->part_cap = 0;
+        HTR_TRY(htr_dev_alloc(dev, part, HTR_MEM_WORK, (void **)&v->part));
+        v->part_cap = part;
     }
     return 0;
 }
@@ -460,7 +472,8 @@ extern "C" int htr_vision_encode(htr_vision *v, const uint8_t *h_rgb, int width,
         }
         // rope2d is applied as K is rounded into its blocks and as the attention reads q
         HTR_TRY(launch_heads_f16(dev, st, v->k, v->v, v->kv, n, c.n_head, v->cs, px, max_pos));
-        HTR_TRY(launch_attn_vision(dev, st, v->q, v->kv, v->a16, n, c.n_head, scale, v->cs, px, max_pos));
+        HTR_TRY(launch_attn_vision(dev, st, v->q, v->kv, v->a16, n, c.n_head, scale, v->cs, px, max_pos,
+                                   v->part));
         HTR_TRY(launch_gemm_f16(dev, st, GEMM_ACC, v->a16, n, l.o, nullptr, v->x, nullptr, 1.0f));
         HTR_TRY(launch_rms_norm_f16(dev, st, v->x, l.ln2, v->h16, n, d, c.eps));
         HTR_TRY(launch_gemm_f16(dev, st, GEMM_FFN, v->h16, n, l.gate, l.up, nullptr, v->g16, 1.0f / FFN_DOWN_SCALE));

@@ -51,6 +51,24 @@ def test_tiny_encoder_on_cut_attention_tiles_matches_oracle(tiny, w, h):
     assert e < 2e-4  # the bar of the tiny encoders' first layer
 
 
+def test_encoder_gives_back_what_a_page_took(dev):
+    """900 patches: 8 attention tiles, all cut along their keys. Their parts, one a worker and one more for each tile but the
+    first, of 256 queries x 68 f32, go with the model as its other buffers do; smaller pages need no more"""
+    cfg = dict(tiny_vision_cfg(), image_size=1540)
+    t = tiny_vision_tensors(cfg)
+    before = dev.mem_live()
+    v = htr.Vision(dev, cfg, t)
+    v.encode(tiny_page(cfg, 420, 420, seed=1), 1)
+    work = dev.mem_live()["work"]
+    parts, workers = (8 - 1) * 256 * 68 * 4, 2 * dev.info()[1] * 256 * 68 * 4
+    assert work - before["work"] < parts + workers + 900 * 80 * cfg["dim"]
+    for w, h in ((392, 420), (28, 28), (420, 420)):
+        v.encode(tiny_page(cfg, w, h, seed=1), 1)
+        assert dev.mem_live()["work"] == work
+    v.free()
+    assert dev.mem_live() == before
+
+
 def test_encoder_keeps_scores_of_two_to_the_27(dev):
     """a page of one colour, q = 8·k and k ~ 1300: every query's largest score is its own key's, 1.0e8 … 1.2e8 of the f32
     values 8 apart, and every value row is the same, so the attention's output is that row whatever the softmax's weights
