@@ -514,15 +514,12 @@ int launch(htr_device *dev, hipStream_t st, int epi, GemmK &a, bool *normed = nu
         }
     }
     // too few 256 / 128 tiles and a long K (one weight; N a multiple of 4): 128 × 128 tiles with K split over up to 4
-    // workgroups (a multiple of 32 each), the products summed in split order by k_split_reduce. A very long K also where
-    // two workgroups a tile are about one a CU (2145 × 1024 × 8192, the projector's merger: 87 → 67 + 6 µs)
+    // workgroups (a multiple of 32 each), the products summed in split order by k_split_reduce
     a.split = 1;
-    if (pick != 0 && epi != GEMM_FFN && a.n_w == 1 && a.rows[0] % 4 == 0 && n_tiles[1] > 0 &&
-        ((n_tiles[1] < want && a.k >= 1024) || (16 * n_tiles[1] <= 9 * dev->n_cu && a.k >= 4096))) {
+    if (pick != 0 && epi != GEMM_FFN && a.n_w == 1 && a.rows[0] % 4 == 0 && n_tiles[1] > 0 && n_tiles[1] < want &&
+        a.k >= 1024) {
         int sp = std::min(4, (dev->n_cu + n_tiles[1] - 1) / n_tiles[1]);
         while (sp > 1 && a.k % (32 * sp)) sp--;
-        // a graph of the caller's keeps no scratch address where the shape has another way
-        if (n_tiles[1] >= want && dev->capturing) sp = 1;
         if (sp > 1) {
             void *part = nullptr;
             HTR_TRY(htr_scratch(dev, SCR_GEMM_PART, (size_t)sp * a.m * a.rows[0] * 4, &part));

@@ -345,6 +345,25 @@ def test_matmul_q8_0_f32_path_over_the_range_of_f32(dev, m, n, k):
     w.free()
 
 
+# a K split over workgroups, and just more tiles than that takes
+@pytest.mark.parametrize("m,n,k", [(1023, 1024, 4096), (2049, 1024, 4096)])
+def test_gemm_f16_recorded_in_a_graph_sums_as_the_direct_call(dev, m, n, k):
+    w = htr.Weight(dev, htr.synth_q8_0(31, n, k), n, k, f16=True)
+    xb, y = dev.upload(htr.synth_normal(32, m * k).astype(np.float16)), dev.alloc(m * n * 4)
+    htr.gemm_f16(dev, xb, m, w, y)
+    eager = y.download(np.float32)
+    dev.capture_begin()
+    htr.gemm_f16(dev, xb, m, w, y)
+    g = dev.capture_end()
+    for rep in range(3):
+        y.upload(np.full(m * n, np.nan, np.float32))
+        g.launch()
+        dev.sync()
+        assert np.array_equal(y.download(np.float32), eager), rep
+    g.free()
+    w.free()
+
+
 # one block; an odd block count; row counts around the tile of 32; the decoder's width
 @pytest.mark.parametrize("n_tok,dim,n_kv", [(1, 32, 1), (31, 96, 2), (33, 160, 1), (65, 1024, 2)])
 def test_f32_prefill_values_are_the_reference_fma_chain(dev, n_tok, dim, n_kv):
