@@ -458,9 +458,9 @@ __global__ __launch_bounds__(AW) void k_attn_decode(const float *q, const _Float
 // attention_causal.wgsl's arithmetic (text.rs:484-499; the same on every compute path): q·scale in f32, scores as
 // f32 dot products with the f16 keys, an online softmax in f32 over the keys each query sees (0 … its position),
 // out = acc · (1 / l). Here on the f16 matrix cores (v_mfma_f32_32x32x16_f16) with f32-grade operands: q·scale =
-// qh + ql and p·2^10 = ph + pl, each half rounded to f16 (K and V are f16 already), so every product of what is held is
-// exact and every sum f32; the 2^10 (exact) drops out with l, which carries it too. The p pair holds 22 bits of p down to
-// 2^-12 of a query's largest, and is within 2^-35 of that largest below (pl is subnormal there). The q pair holds 22 bits,
+// qh + ql and 2^3·p = ph + pl, each half rounded to f16 (K and V are f16 already), so every product of what is held is
+// exact and every sum f32; the 2^3 (exact) drops out with l, which carries it too. The p pair holds 22 bits of p down to
+// 2^-5 of a query's largest, and is within 2^-28 of that largest below (pl is subnormal there). The q pair holds 22 bits,
 // except that qh is rounded from the f32 product and ql is the rest beside the product rounded to f16 in one step (that
 // is how the compiler takes x·scale where both are wanted): where the f32 product is a tie the two f16 values differ, and
 // the pair is an f16 ulp off (5e-5 of random elements, none with a power of two as scale; the outputs' error against 64
@@ -478,10 +478,12 @@ __global__ __launch_bounds__(AW) void k_attn_decode(const float *q, const _Float
 //            on different bank groups. Keys past the last read the last key and are masked;
 //   scores   Sᵀ (32 keys × 32 queries) = K·(qh + ql)ᵀ: lane ℓ = 32h + c holds query c's scores of keys
 //            8(i / 4) + 4h + i % 4 (i < 16); the max over a query's keys is one swap across lane bit 5;
-//   softmax  p = 2^(s·log2 e + nm), nm = 10 − log2 e · (the max when it was last moved): one fma and one v_exp_f32 a
+//   softmax  p = 2^(s·log2 e + nm), nm = 3 − log2 e · (the max when it was last moved): one fma and one v_exp_f32 a
 //            score, and nm is the only state, so its rounding cancels between p, l and O. nm moves (and O and l are
-//            rescaled) only when some p would pass 2^15, so most blocks skip the 64-register rescale. nm holds scores of
-//            2^26 to within 4, and p to 2^14 with them; a wave with a query whose scores could be larger (Σ |q·scale| of
+//            rescaled) only when some p would pass 2^8, so most blocks skip the 64-register rescale. An exponent is
+//            rounded at its own size, which is why the shift is small (10, and 15 for the top: 2.3e-7 against 64 bits
+//            for 64 queries, 2.9e-7 for 1925; 1.9e-7 and 2.4e-7 so, as e^(s − max) gave), and l is summed a block at a
+//            time, for the same reason. nm holds scores of 2^26 to within 4, so p keeps to f16's range; a wave with a query whose scores could be larger (Σ |q·scale| of
 //            a half row from 512 on, against f16 keys of 65504 at most) keeps the max itself and takes s − max first;
 //   values   Oᵀ (128 dims × 32 queries) += Vᵀ·(ph + pl)ᵀ: the Vᵀ operand by ds_read_b64_tr_b16 (16 lanes read 4 key
 //            rows × 16 dims and each gets one dim's 4 keys), the P operand straight from the lane's score registers.
@@ -495,7 +497,7 @@ __global__ __launch_bounds__(AW) void k_attn_decode(const float *q, const _Float
 // 2000 earlier keys gained, 31.4 → 29.7.
 constexpr int CQ = 32, CK = 32, CB_CHUNKS = 1024;  // queries a workgroup, keys a block, 16-byte chunks a key block
 constexpr int CKS = 2, CW = 64 * 2 * CKS;          // key parts; threads
-constexpr float P_SHIFT = 10.0f, P_TOP = 15.0f;    // log2 of the largest p when nm moves, and before it must
+constexpr float P_SHIFT = 3.0f, P_TOP = 8.0f;      // log2 of the largest p when nm moves, and before it must
 constexpr float LOG2E = 1.4426950408889634f;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -671,6 +673,7 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
             return v;
         };
         uint32_t ph[8], pl[8];
+        float ls;
         half8 a[8], v[4];
 #pragma unroll
         for (int ks = 0; ks < 3; ks++) a[ks] = *reinterpret_cast<const half8 *>(kb + ka[ks]);
@@ -687,14 +690,15 @@ __global__ __launch_bounds__(CW) void k_attn_causal(const float *q, const _Float
             asm volatile("" : "+v"(ph[ks]));  // holds the conversion here
             __builtin_amdgcn_sched_barrier(0);
             sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks], ql[ks], sn, 0, 0, 0);
-            l += p[0];
-            l += p[1];
+            ls = ks ? ls + p[0] : p[0];
+            ls += p[1];
             const half2_t lo = __builtin_convertvector((float2_t{minus_half<0>(p[0], ph[ks]), minus_half<1>(p[1], ph[ks])}), half2_t);
             __builtin_memcpy(&pl[ks], &lo, 4);
             asm volatile("" : "+v"(pl[ks]));
             __builtin_amdgcn_sched_barrier(0);
         }
         v[3] = vread(3, 0);
+        l += ls;
 #pragma unroll
         for (int ss = 0; ss < 2; ss++) {
             half8 h8, l8;

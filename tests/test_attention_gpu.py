@@ -240,3 +240,23 @@ def test_causal_attention_of_scores_up_to_two_to_the_31(dev, n_q, pos0):
     for i in range(n_q):
         row = orc.attn_f64(q[i * n_head:(i + 1) * n_head].ravel(), k, v, 128, pos0 + i + 1, n_head, n_kv, 0.125)
         assert rel_l2(got[i], row) < 1e-5, i
+
+
+def test_causal_attention_weights_of_two_keys_to_f32(dev):
+    """the ratio of two keys' weights against e^(difference) in 64 bits: scores 0 and -d, exact, d up to 1.3; values 1 in
+    one half of the dims and 0 in the other. Bar, rms over 2048 queries: an exponent under 4 is rounded to 2^-23 at most
+    (4.8e-8 of p), v_exp_f32 and each weight's pair and output to an f32 ulp (3.4e-8 each): 9e-8 in all"""
+    n_kv, rng = 1024, np.random.default_rng(3)
+    d = rng.uniform(0.0, 1.3, 2 * n_kv).astype(np.float32)
+    k, v = np.zeros((n_kv, 2, 128), np.float16), np.zeros((n_kv, 2, 128), np.float16)
+    k[:, 1, 0], v[:, 0, :64], v[:, 1, 64:] = -1.0, 1.0, 1.0
+    q = np.zeros((2 * n_kv, 128), np.float32)
+    q[:, 0] = 8 * d
+    # two f16 values hold 22 of a score's 24 bits: those the kernel works with
+    s = (q[:, 0] * np.float32(0.125)).astype(np.float32)
+    held = s.astype(np.float16).astype(np.float64) + (s - s.astype(np.float16).astype(np.float32)).astype(np.float16)
+    out = dev.alloc(q.nbytes)
+    htr.causal_attention(dev, dev.upload(q), dev.upload(k), dev.upload(v), 1, 1, 2 * n_kv, n_kv, 2, 0.125, out)
+    o = out.download(np.float32).reshape(-1, 128).astype(np.float64)
+    err = (o[:, 64] / o[:, 0]) / np.exp(-held) - 1.0
+    assert np.sqrt(np.mean(err ** 2)) < 1.2e-7
