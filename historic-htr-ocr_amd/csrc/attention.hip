@@ -483,8 +483,9 @@ __global__ __launch_bounds__(AW) void k_attn_decode(const float *q, const _Float
 //            rescaled) only when some p would pass 2^8, so most blocks skip the 64-register rescale. An exponent is
 //            rounded at its own size, which is why the shift is small (10, and 15 for the top: 2.3e-7 against 64 bits
 //            for 64 queries, 2.9e-7 for 1925; 1.9e-7 and 2.4e-7 so, as e^(s − max) gave), and l is summed a block at a
-//            time, for the same reason. nm holds scores of 2^26 to within 4, so p keeps to f16's range; a wave with a query whose scores could be larger (Σ |q·scale| of
-//            a half row from 512 on, against f16 keys of 65504 at most) keeps the max itself and takes s − max first;
+//            time, for the same reason. nm holds scores of 2^26 to within 4, so p keeps to f16's range; a wave with a
+//            query whose scores could be larger (Σ |q·scale| of a half row from 512 on, against f16 keys of 65504 at
+//            most) keeps the max itself and takes s − max first;
 //   values   Oᵀ (128 dims × 32 queries) += Vᵀ·(ph + pl)ᵀ: the Vᵀ operand by ds_read_b64_tr_b16 (16 lanes read 4 key
 //            rows × 16 dims and each gets one dim's 4 keys), the P operand straight from the lane's score registers.
 //
