@@ -692,9 +692,11 @@ template <bool EX> int gemm_q8(htr_device *dev, hipStream_t st, const float *x, 
         return htr_launched(dev, EX ? "k_gemm_q8_0_few<f32>" : "k_gemm_q8_0_few<f16>");
     }
     // 128 × 128 tiles from one a CU on; of the 64 × 64 ones, 4 K groups while every CU has a tile at most, else 2, whose
-    // workgroups go two to a CU (288 tiles, 333 × 3072 × 1024: f16 18.5 → 14.2 µs, F32 24.1 → 21.8)
+    // workgroups go two to a CU (288 tiles, 333 × 3072 × 1024: f16 18.5 → 14.2 µs, F32 24.1 → 21.8); 2 for a short K too,
+    // where a group has a stage or two and the sum of four costs more than they save (4 → 2 groups, 100 × 1024: F32
+    // K = 64 5.0 → 4.3, 256 6.1 → 6.0, 384 7.1 → 7.2; f16 K = 64 6.0 → 4.5, 512 6.9 → 6.3)
     if (t128 >= dev->n_cu) launch_q8<EX, 2, 1>(dev, st, x, w, y, m, acc);
-    else if (t64 > dev->n_cu) launch_q8<EX, 1, 2>(dev, st, x, w, y, m, acc);
+    else if (t64 > dev->n_cu || w->cols <= (EX ? 256 : 512)) launch_q8<EX, 1, 2>(dev, st, x, w, y, m, acc);
     else launch_q8<EX, 1, 4>(dev, st, x, w, y, m, acc);
     return htr_launched(dev, EX ? "k_gemm_q8_0<f32>" : "k_gemm_q8_0<f16>");
 }

@@ -238,7 +238,7 @@ def _deq64(blocks, n, k):
 # one block, odd block counts, tiles of 64 and 128 cut on both sides; the tile counts on either side of the launch's
 # rules (4 K groups, 2 K groups, 128 × 128 tiles); X off the 16-byte grid
 @pytest.mark.parametrize("m,n,k,off", [(1, 1, 32, 0), (1, 65, 96, 4), (63, 129, 160, 0), (64, 64, 64, 8), (65, 63, 1024, 0),
-                                       (333, 1000, 3072, 0), (1025, 2000, 224, 0), (2050, 2049, 96, 0), (2050, 2049, 64, 4)])
+                                       (333, 1000, 3072, 0), (65, 129, 544, 4), (1025, 2000, 224, 0), (2050, 2049, 96, 0), (2050, 2049, 64, 4)])
 def test_matmul_q8_0_tiles_against_fp64(dev, m, n, k, off):
     """every output within the f32 rounding of its own sum: K/32 block sums added one by one (and, on the F32 path, a
     block's 3 · 32 exact products before them; on the f16 path the K products)"""
