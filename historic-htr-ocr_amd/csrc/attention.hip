@@ -492,10 +492,11 @@ __global__ __launch_bounds__(AW) void k_attn_decode(const float *q, const _Float
 // Bound: the score MFMAs with the softmax between them (a 32x32x16 MFMA takes 17 ns a SIMD here; with its 5 VALU
 // instructions and exponential about 23), then the stage's loads (20 %: a timing copy without them ran 34 µs for 40) and
 // a stage's barrier. Measured against 16 queries a workgroup on 16x16x32 MFMAs, O rescaled at every block and the keys
-// copied into blocks by a launch before it (n_q from position 0, 16 / 8 heads, µs a kernel): 333 queries 11.5 + 4.9 →
-// 10.5, 1023 26.0 + 5.5 → 21.9, 1925 75.6 + 8.1 → 40.5 (375 TFLOP/s of q·k and p·v). Eight waves and four key parts, one
-// workgroup a CU: 13.7, 23.4, 48.6 (its merge is twice the LDS traffic and its waves run in step); only 32 queries on
-// 2000 earlier keys gained, 31.4 → 29.7.
+// copied into blocks by a launch before it (n_q from position 0, 16 / 8 heads, median µs of a kernel trace): 1925 queries
+// 75.2 + 8.0 → 42.9 (39.6 a call among others: 383 TFLOP/s of q·k and p·v); with the q heads' norm and RoPE, which a third
+// launch did (5.2 and 9.4 with the K / V rows, now 4.8 and 5.1): 333 11.4 + 4.9 → 13.1, 1023 25.9 + 5.5 → 24.4.
+// Eight waves and four key parts, one workgroup a CU: 20 % slower at 1925 queries (its merge is twice the LDS traffic and
+// its waves run in step); only 32 queries on 2000 earlier keys gained, 31.4 → 29.7.
 constexpr int CQ = 32, CK = 32, CB_CHUNKS = 1024;  // queries a workgroup, keys a block, 16-byte chunks a key block
 constexpr int CKS = 2, CW = 64 * 2 * CKS;          // key parts; threads
 constexpr float P_SHIFT = 3.0f, P_TOP = 8.0f;      // log2 of the largest p when nm moves, and before it must

@@ -50,11 +50,12 @@ __global__ __launch_bounds__(256) void k_swiglu(float *g, const float *u, size_t
 // prompt of some hundred rows makes few tiles, and the groups give such a CU four waves a SIMD to hide the loads'
 // latency without a second launch for the sum. A stage is KB blocks of 32 k (f16: 2, EX: 1); its loads go to registers
 // R stages ahead and are converted as they are stored to LDS (16-byte chunks of 8 k, XOR-placed so that the 16 lanes of
-// a fragment read fall on 16 bank groups). K past the last block is zeros, rows past M and columns past N are read clamped and not stored.
+// a fragment read fall on 16 bank groups). K past the last block is zeros, rows past M and columns past N are read clamped
+// and not stored.
 // Bound: the 128 × 128 tile's MFMAs and conversions about even; the 64 × 64 ones by the stages' load latency. Measured
 // against the kernels before it (f32 FMA tiles on the f16 path, v_mfma_f32_32x32x2_f32 on the F32 path), a call: f16
-// 48 × 1024 × 2048 231 → 13.4 µs, 1925 × 3072 × 1024 422 → 30.4 µs (399 TFLOP/s); F32 1023 × 1024 × 3072 onto the
-// residual 111 → 35 µs (185 TFLOP/s, past the f32 MFMA's 157 peak). Error against 64 bits 5.6e-7 … 9.8e-7 → 1.2e-7 …
+// 48 × 1024 × 2048 230 → 13.2 µs, 1925 × 3072 × 1024 422 → 29.8 µs (406 TFLOP/s); F32 1023 × 1024 × 3072 onto the
+// residual 111 → 35 µs (182 TFLOP/s, past the f32 MFMA's 157 peak). Error against 64 bits 5.6e-7 … 9.8e-7 → 1.2e-7 …
 // 2.0e-7: a block's 96 products are summed inside the matrix unit before the one f32 fma that scales them.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -109,7 +110,8 @@ __device__ __forceinline__ void split3(const float (&x)[8], int4 (&out)[3], Q8Se
 // quants (q · 2^e is a bf16 value) and m = 1 … 2, with d's sign, on the block's sum. ±inf, NaN, d = ±inf and NaN as the
 // products q·d·x give them. The products and their order are those of the caller's own pass (ko, kh: where the lane's first
 // 8 k of a block start, and its other 8), so a row's results do not depend on the other rows. Straight from memory, one
-// block at a time: a tile that needs it takes several times as long
+// block at a time: a tile that needs it takes several times as long. (The matrix unit keeps subnormal bf16 operands and
+// f32 sums.)
 __device__ __forceinline__ f32x16 wide_blocks(const float *x, const int8_t *q, const _Float16 *d, int b0, int b1, int step,
                                               int ko, int kh) {
     typedef uint16_t ushort8 __attribute__((ext_vector_type(8)));
@@ -528,11 +530,11 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void k_gemm_q8_0_few(const float *x
 // Y = X·Wᵀ with every output one chain of f32 fmas over k in order (matmul.wgsl:47-91), bit for bit: v_mfma_f32_16x16x4_f32
 // adds its four products one after another, each rounded. K and V are rounded to f16 into the cache, where a last-bit
 // difference of the f32 sum can move a value by an f16 ulp, which then stays in every later layer: with these two products
-// in the reference's order the logits of a 1023-token prompt through 28 layers are 4.5e-5 from the f32 oracle's, with the
-// exact block sums of k_gemm_q8_0 (which no order of f32 sums equals) 1.15e-4.
+// in the reference's order the logits of a 1023-token prompt through 28 layers are 4.6e-5 from the f32 oracle's, with the
+// exact block sums of k_gemm_q8_0 (which no order of f32 sums equals) 1.16e-4.
 // A workgroup owns 32 × 64 outputs of one of the two matrices (grid z), 4 waves of 16 × 32; K in stages of two q8_0
-// blocks, double-buffered in LDS as f32, their loads two stages ahead. A row's 32 values lie by k mod 4, then k / 4, so a lane's operands of the 8 MFMAs (k = 4s
-// + its quarter) are two 16-byte chunks, placed at chunk ^ (row/2 % 8). Bound: the
+// blocks, double-buffered in LDS as f32, their loads two stages ahead. A row's 32 values lie by k mod 4, then k / 4, so a
+// lane's operands of the 8 MFMAs (k = 4s + its quarter) are two 16-byte chunks, placed at chunk ^ (row/2 % 8). Bound: the
 // stages' latency at prompt sizes (333 × 2 · 1024 × 1024 28.7 µs a launch, 49 TFLOP/s; one block a stage 33.5 µs).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
