@@ -104,56 +104,93 @@ __device__ __forceinline__ void split3(const float (&x)[8], int4 (&out)[3], Q8Se
     for (int s = 0; s < 3; s++) out[s] = hi_halves(b[s]);
 }
 
-// 32 × 32 outputs of a wave over the blocks b0, b0 + step, … below b1, each product exact for all of f32 and a block's sum
+// 32 × 32J outputs of a wave over the blocks b0, b0 + step, … below b1, each product exact for all of f32 and a block's sum
 // finite where the scaled one is: x = b1 + 2^-8·b2 + 2^-16·b3, what is left scaled up each time (it is under 2^-7·|x|), so
 // that nothing is lost at the lower end, against the quants with 2^0, 2^-8 and 2^-16; and d = 2^e · m, with 2^e on the
 // quants (q · 2^e is a bf16 value) and m = 1 … 2, with d's sign, on the block's sum. ±inf, NaN, d = ±inf and NaN as the
-// products q·d·x give them. The products and their order are those of the caller's own pass (ko, kh: where the lane's first
-// 8 k of a block start, and its other 8), so a row's results do not depend on the other rows. Straight from memory, one
-// block at a time: a tile that needs it takes several times as long. (The matrix unit keeps subnormal bf16 operands and
-// f32 sums.)
-__device__ __forceinline__ f32x16 wide_blocks(const float *x, const int8_t *q, const _Float16 *d, int b0, int b1, int step,
-                                              int ko, int kh) {
+// products q·d·x give them. (The matrix unit keeps subnormal bf16 operands and f32 sums.) The products and their order are
+// those of the caller's own pass (q, d: the J weight rows; ko, kh: where the lane's first 8 k of a block start, and its
+// other 8), so a row's results do not depend on the other rows. Straight from memory, a block at a time: 1023 × 1024 × 3072
+// with a subnormal value (a SwiGLU output, say) in one row 35 → 105 µs, in every row 110
+template <int J>
+__device__ __forceinline__ void wide_blocks(const float *x, const int8_t *const (&q)[J], const _Float16 *const (&d)[J],
+                                            int b0, int b1, int step, int ko, int kh, int al, f32x16 (&c)[J]) {
     typedef uint16_t ushort8 __attribute__((ext_vector_type(8)));
-    f32x16 c = {};
-#pragma unroll 1
-    for (int b = b0; b < b1; b += step) {
-        const float ds = (float)d[b];
-        const float pow2 = fmaxf(__uint_as_float(__float_as_uint(ds) & 0x7f800000u), 0x1p-24f);  // of 0: m is 0
-        const float mant = __uint_as_float((__float_as_uint(ds) & 0x807fffffu) | 0x3f800000u);
-        f32x16 p = {};
+    struct Regs {
+        float4 a[2][2];
+        int2 q[J][2];
+        _Float16 d[J];
+    };
+    auto gload = [&](int b) {
+        Regs r;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int at = 32 * b + ko + h * kh;
-            uint32_t f[3][8], w[8];
+            const float *xs = x + at;
+            if (al) {
+                r.a[h][0] = reinterpret_cast<const float4 *>(xs)[0];
+                r.a[h][1] = reinterpret_cast<const float4 *>(xs)[1];
+            } else {
+                r.a[h][0] = make_float4(xs[0], xs[1], xs[2], xs[3]);
+                r.a[h][1] = make_float4(xs[4], xs[5], xs[6], xs[7]);
+            }
+#pragma unroll
+            for (int j = 0; j < J; j++) r.q[j][h] = *reinterpret_cast<const int2 *>(q[j] + at);
+        }
+#pragma unroll
+        for (int j = 0; j < J; j++) r.d[j] = d[j][b];
+        return r;
+    };
+#pragma unroll
+    for (int j = 0; j < J; j++) c[j] = f32x16{};
+#pragma unroll 1
+    for (int b = b0; b < b1; b += step) {
+        const Regs r = gload(b);
+        f32x16 p[J] = {};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float4 u = r.a[h][0], v = r.a[h][1];
+            const float xv[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+            uint32_t f[3][8];
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                const float v = x[at + e], r1 = (v - __uint_as_float(__float_as_uint(v) & 0xffff0000u)) * 256.0f;
+                f[0][e] = __float_as_uint(xv[e]);
+                const float r1 = (xv[e] - __uint_as_float(f[0][e] & 0xffff0000u)) * 256.0f;
                 const float r2 = (r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u)) * 256.0f;
-                const bool inf = fabsf(v) == INFINITY;  // inf − inf would make NaN of it
-                f[0][e] = __float_as_uint(v);
+                const bool inf = fabsf(xv[e]) == INFINITY;  // inf − inf would make NaN of it
                 f[1][e] = inf ? 0u : __float_as_uint(r1);
                 f[2][e] = inf ? 0u : __float_as_uint(r2);
-                w[e] = __float_as_uint((float)q[at + e] * pow2);
             }
-            ushort8 wb;
-            const int4 w4 = hi_halves(w);
-            __builtin_memcpy(&wb, &w4, 16);
 #pragma unroll
-            for (int pl = 0; pl < 3; pl++) {
-                if (pl) wb = __builtin_elementwise_sub_sat(wb, (ushort8)(uint16_t)(8 << 7));  // 8 off each exponent; a 0 stays
-                const int4 a4 = hi_halves(f[pl]);
-                bf16x8 a, wp;
-                __builtin_memcpy(&a, &a4, 16);
-                __builtin_memcpy(&wp, &wb, 16);
-                p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wp, p, 0, 0, 0);
+            for (int j = 0; j < J; j++) {
+                // 2^e of d (of 0: the smallest, m is 0)
+                const float pow2 = fmaxf(__uint_as_float(__float_as_uint((float)r.d[j]) & 0x7f800000u), 0x1p-24f);
+                uint32_t w[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) w[e] = __float_as_uint((float)q_byte(r.q[j][h], e) * pow2);
+                const int4 w4 = hi_halves(w);
+                ushort8 wb;
+                __builtin_memcpy(&wb, &w4, 16);
+#pragma unroll
+                for (int pl = 0; pl < 3; pl++) {
+                    // 8 off each exponent; a zero stays
+                    if (pl) wb = __builtin_elementwise_sub_sat(wb, (ushort8)(uint16_t)(8 << 7));
+                    const int4 a4 = hi_halves(f[pl]);
+                    bf16x8 a, wp;
+                    __builtin_memcpy(&a, &a4, 16);
+                    __builtin_memcpy(&wp, &wb, 16);
+                    p[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wp, p[j], 0, 0, 0);
+                }
             }
         }
-        const float m = ds == 0.0f || ds != ds ? ds : mant;
 #pragma unroll
-        for (int i = 0; i < 16; i++) c[i] = fmaf(p[i], m, c[i]);
+        for (int j = 0; j < J; j++) {
+            const float ds = (float)r.d[j];
+            const float m = ds == 0.0f || ds != ds ? ds : __uint_as_float((__float_as_uint(ds) & 0x807fffffu) | 0x3f800000u);
+#pragma unroll
+            for (int i = 0; i < 16; i++) c[j][i] = fmaf(p[j][i], m, c[j][i]);
+        }
     }
-    return c;
 }
 
 template <bool EX, int T, int KG> struct Q8Tile {
@@ -339,13 +376,16 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q8_0(const float *x, const in
         if (__builtin_amdgcn_ballot_w64(seen.wide()) && lane == 0) s_wide = 1;
         __syncthreads();
         if (__builtin_expect(s_wide, 0)) {
+            const int8_t *qs[T];
+            const _Float16 *ds[T];
+#pragma unroll
+            for (int j = 0; j < T; j++) {
+                const size_t wr = min(col0 + fb + 32 * j, n - 1);
+                qs[j] = wq + wr * k, ds[j] = wd + wr * nb;
+            }
 #pragma unroll
             for (int i = 0; i < T; i++)
-#pragma unroll
-                for (int j = 0; j < T; j++) {
-                    const size_t xr = min(row0 + fa + 32 * i, m - 1), wr = min(col0 + fb + 32 * j, n - 1);
-                    c[i][j] = wide_blocks(x + xr * k, wq + wr * k, wd + wr * nb, grp, nb, KG, 8 * hk, 16);
-                }
+                wide_blocks<T>(x + (size_t)min(row0 + fa + 32 * i, m - 1) * k, qs, ds, grp, nb, KG, 8 * hk, 16, al, c[i]);
         }
     }
     // lane ℓ, register r: row 8(r/4) + 4(ℓ/32) + r%4, column ℓ%32 of each 32 × 32 tile
@@ -500,8 +540,13 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void k_gemm_q8_0_few(const float *x
                 gload(ring[i], i0 + i + FEW_R);
             }
     }
-    if (EX && __builtin_expect(__builtin_amdgcn_ballot_w64(seen.wide()) != 0, 0))
-        c = wide_blocks(xr, q, d, b0, b1, 1, 0, 8);  // (xr and q start at the lane's half of a block)
+    if (EX && __builtin_expect(__builtin_amdgcn_ballot_w64(seen.wide()) != 0, 0)) {
+        const int8_t *const qs[1] = {q};
+        const _Float16 *const ds[1] = {d};
+        f32x16 wide[1];
+        wide_blocks<1>(xr, qs, ds, b0, b1, 1, 0, 8, al, wide);  // (xr and q start at the lane's half of a block)
+        c = wide[0];
+    }
     // lane ℓ, register r: row 8(r/4) + 4(ℓ/32) + r%4, column ℓ%32
 #pragma unroll
     for (int i = 0; i < 16; i++) s_o[wave][8 * (i >> 2) + 4 * hk + (i & 3)][r32] = c[i];
